@@ -1198,7 +1198,7 @@ static int ibm_enqueue_wide(const FieldsView& v, IbmState* s, void* ring, uint32
     hipLaunchKernelGGL(k_ibm_reset, dim3(nblk(s->K, 64)), dim3(64), 0, st, s->diag, s->K);
     AUXCHK(v, hipGetLastError());
   }
-  const uint32_t gm = nblk((size_t)s->M), gu = nblk(s->U);
+  const uint32_t gu = nblk(s->U);
   const uint32_t gm4 = nblk((size_t)s->M, 4), gu4 = nblk(s->U, 4);  // one wave per marker / cell
   for (int it = 0; it < s->cfg.max_iterations; ++it) {
     if (record && s->U)

@@ -137,6 +137,47 @@ struct ProbeArgs {
   float* out;      // 3: the step's probed force
 };
 
+// Collide-stream launchers of one lattice, storage and collision (KIND 0
+// TRT/BGK, 1 central moments), specialised in lbm_hydro.hip, one object file
+// each; list: the force-listed cells instead of the tiles.
+template <int Q, int STORAGE, int KIND>
+hipError_t hydro_launch(int odd, const HydroArgs& a, hipStream_t s, bool list);
+template <int Q, int STORAGE, int KIND>
+hipError_t batch_launch(int odd, const HydroArgs* tab, const uint32_t* ent, uint32_t nent, uint32_t grid,
+                        const uint32_t* cells, uint32_t ncells, hipStream_t s);
+#define LBM_DECL_HYDRO(Q, S, K)                                                                    \
+  template <>                                                                                      \
+  hipError_t hydro_launch<Q, S, K>(int odd, const HydroArgs& a, hipStream_t s, bool list);         \
+  template <>                                                                                      \
+  hipError_t batch_launch<Q, S, K>(int odd, const HydroArgs* tab, const uint32_t* ent,             \
+                                   uint32_t nent, uint32_t grid, const uint32_t* cells, uint32_t ncells, \
+                                   hipStream_t s);
+#define LBM_DECL_HYDRO_S(Q) \
+  LBM_DECL_HYDRO(Q, kF32, 0) LBM_DECL_HYDRO(Q, kF32, 1) LBM_DECL_HYDRO(Q, kF16, 0) \
+  LBM_DECL_HYDRO(Q, kF16, 1) LBM_DECL_HYDRO(Q, kBF16, 0) LBM_DECL_HYDRO(Q, kBF16, 1)
+LBM_DECL_HYDRO_S(19)
+LBM_DECL_HYDRO_S(27)
+// Open faces and volume sources of one lattice and storage (specialised in
+// lbm_open.hip, one object file each).
+template <int Q, int STORAGE>
+hipError_t open_launch(const FaceArgs& a, hipStream_t s);
+template <int Q, int STORAGE>
+hipError_t source_launch(const SourceArgs& a, hipStream_t s);
+#define LBM_DECL_OPEN(Q, S)                                       \
+  template <>                                                     \
+  hipError_t open_launch<Q, S>(const FaceArgs& a, hipStream_t s); \
+  template <>                                                     \
+  hipError_t source_launch<Q, S>(const SourceArgs& a, hipStream_t s);
+LBM_DECL_OPEN(19, kF32)
+LBM_DECL_OPEN(19, kF16)
+LBM_DECL_OPEN(19, kBF16)
+LBM_DECL_OPEN(27, kF32)
+LBM_DECL_OPEN(27, kF16)
+LBM_DECL_OPEN(27, kBF16)
+#undef LBM_DECL_OPEN
+#undef LBM_DECL_HYDRO_S
+#undef LBM_DECL_HYDRO
+
 // Host-side launchers (lbm_kernels.hip).  All enqueue on `s`.
 hipError_t launch_hydro(int Q, int storage, int collision, int odd, const HydroArgs& a, hipStream_t s);
 hipError_t launch_hydro_list(int Q, int storage, int collision, int odd, const HydroArgs& a, hipStream_t s);

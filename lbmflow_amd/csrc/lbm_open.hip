@@ -32,7 +32,8 @@
 // thread reads what another writes, so one launch does all three per cell.
 // The stash is double-buffered and starts at zero (the reference's ftmp).
 // Face kernels are templated on the face so every lattice direction is a
-// compile-time constant (no indexed register arrays).
+// compile-time constant (no indexed register arrays).  The file is compiled
+// once per lattice and storage (LBM_Q, LBM_STORAGE as in lbm_hydro.hip).
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
 
@@ -456,89 +457,46 @@ __global__ __launch_bounds__(256) void k_volume_source(SourceArgs a) {
   });
 }
 
-hipError_t launch_volume_source(int Q, int storage, const SourceArgs& a, hipStream_t s) {
-  const uint32_t n = (a.hi[0] - a.lo[0] + 1) * (a.hi[1] - a.lo[1] + 1) * (a.hi[2] - a.lo[2] + 1);
-  const dim3 g((n + 255) / 256), b(256);
-  if (storage == kF32) {
-    if (Q == 19)
-      hipLaunchKernelGGL((k_volume_source<19, float>), g, b, 0, s, a);
-    else
-      hipLaunchKernelGGL((k_volume_source<27, float>), g, b, 0, s, a);
-  } else if (storage == kF16) {
-    if (Q == 19)
-      hipLaunchKernelGGL((k_volume_source<19, _Float16>), g, b, 0, s, a);
-    else
-      hipLaunchKernelGGL((k_volume_source<27, _Float16>), g, b, 0, s, a);
-  } else {
-    if (Q == 19)
-      hipLaunchKernelGGL((k_volume_source<19, bf16s>), g, b, 0, s, a);
-    else
-      hipLaunchKernelGGL((k_volume_source<27, bf16s>), g, b, 0, s, a);
-  }
-  return hipGetLastError();
-}
-
-// fluid cells of non-periodic faces that no open face covers
-__global__ void k_uncovered(Dom d, const uint8_t* solid, uint32_t open_bits, unsigned int* count) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N || solid[i]) return;
-  uint32_t x, y, z;
-  cell_xyz(d, i, x, y, z);
-  const uint32_t c[3] = {x, y, z}, n[3] = {d.nx, d.ny, d.nz};
-  bool bad = false;
-  for (int ax = 0; ax < 3; ++ax) {
-    if (d.per[ax]) continue;
-    if (c[ax] == 0 && !((open_bits >> (2 * ax)) & 1u)) bad = true;
-    if (c[ax] == n[ax] - 1 && !((open_bits >> (2 * ax + 1)) & 1u)) bad = true;
-  }
-  if (bad) atomicAdd(count, 1u);
-}
-
 static uint32_t max_face_cells(const Dom& d) {
   const uint32_t a = d.ny * d.nz, b = d.nx * d.nz, c = d.nx * d.ny;
   return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
-template <typename S>
-static hipError_t open_s(int Q, const FaceArgs& a, hipStream_t s) {
+template <int Q, typename S>
+static hipError_t open_q(const FaceArgs& a, hipStream_t s) {
   if (a.nfaces == 0) return hipSuccess;
   const dim3 block(256), grid((max_face_cells(a.d) + 255) / 256, (unsigned)a.nfaces);
   bool one_axis = true;
   for (int k = 1; k < a.nfaces; ++k) one_axis = one_axis && a.faces[k] / 2 == a.faces[0] / 2;
   if (one_axis) {
-    if (Q == 19)
-      hipLaunchKernelGGL((k_face_bc<19, S, true>), grid, block, 0, s, a, 0);
-    else
-      hipLaunchKernelGGL((k_face_bc<27, S, true>), grid, block, 0, s, a, 0);
+    hipLaunchKernelGGL((k_face_bc<Q, S, true>), grid, block, 0, s, a, 0);
     return hipGetLastError();
   }
-  if (Q == 19) {
-    hipLaunchKernelGGL((k_face_stash<19, S, false>), grid, block, 0, s, a);
-    hipLaunchKernelGGL((k_face_stash<19, S, true>), grid, block, 0, s, a);
-  } else {
-    hipLaunchKernelGGL((k_face_stash<27, S, false>), grid, block, 0, s, a);
-    hipLaunchKernelGGL((k_face_stash<27, S, true>), grid, block, 0, s, a);
-  }
-  for (int k = 0; k < a.nfaces; ++k) {
-    const int face = a.faces[k];
-    const dim3 g1((max_face_cells(a.d) + 255) / 256);
-    if (Q == 19)
-      hipLaunchKernelGGL((k_face_bc<19, S, false>), g1, block, 0, s, a, face);
-    else
-      hipLaunchKernelGGL((k_face_bc<27, S, false>), g1, block, 0, s, a, face);
-  }
+  hipLaunchKernelGGL((k_face_stash<Q, S, false>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((k_face_stash<Q, S, true>), grid, block, 0, s, a);
+  for (int k = 0; k < a.nfaces; ++k)
+    hipLaunchKernelGGL((k_face_bc<Q, S, false>), dim3(grid.x), block, 0, s, a, a.faces[k]);
   return hipGetLastError();
 }
 
-hipError_t launch_open_faces(int Q, int storage, const FaceArgs& a, hipStream_t s) {
-  if (storage == kF32) return open_s<float>(Q, a, s);
-  if (storage == kF16) return open_s<_Float16>(Q, a, s);
-  return open_s<bf16s>(Q, a, s);
+// this object file's lattice and storage
+#if LBM_STORAGE == 0
+using OpenS = float;
+#elif LBM_STORAGE == 1
+using OpenS = _Float16;
+#else
+using OpenS = bf16s;
+#endif
+
+template <>
+hipError_t open_launch<LBM_Q, LBM_STORAGE>(const FaceArgs& a, hipStream_t s) {
+  return open_q<LBM_Q, OpenS>(a, s);
 }
 
-hipError_t launch_uncovered(const Dom& d, const uint8_t* solid, uint32_t open_bits, unsigned int* count,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(k_uncovered, dim3((d.N + 255) / 256), dim3(256), 0, s, d, solid, open_bits, count);
+template <>
+hipError_t source_launch<LBM_Q, LBM_STORAGE>(const SourceArgs& a, hipStream_t s) {
+  const uint32_t n = (a.hi[0] - a.lo[0] + 1) * (a.hi[1] - a.lo[1] + 1) * (a.hi[2] - a.lo[2] + 1);
+  hipLaunchKernelGGL((k_volume_source<LBM_Q, OpenS>), dim3((n + 255) / 256), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
