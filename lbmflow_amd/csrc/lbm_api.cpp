@@ -444,6 +444,29 @@ int rebuild_mask(lbm_fields* fl) {
   return rebuild_tiles(fl);
 }
 
+// How the tile blocks are dealt to the XCDs (xcd_remap).  A domain whose
+// populations are a few times the last-level cache goes through memory as one
+// stretch per XCD: what a step leaves in that XCD's L2 and in the last level
+// is what its next step reads (64^3 D3Q19 fp32 step: 13.4 us, 15.0 us with
+// short runs; 200^3 D3Q27 fp32: 0.311, 0.322 ms).  Larger domains stream, and
+// eight distant stretches cost DRAM page hits there: short runs keep the XCDs
+// together.  Medians per parity (even / odd ms), one stretch per XCD -> rule:
+//   512^3 tank D3Q27 fp32   4.03 / 4.51 -> 4.01 / 4.35
+//   512^3 tank D3Q27 fp16   2.42 / 2.75 -> 2.31 / 2.73
+//   320^3 tank D3Q19 fp32   0.845 / 0.926 -> 0.825 / 0.894
+//   384 x 256 x 256 periodic D3Q27 fp16  0.591 / 0.717 -> 0.515 / 0.721
+// The odd step's x-shifted rows share lines between neighbouring tiles, so it
+// keeps long runs; 16-bit even steps, whose tile is one line per plane, are
+// best nearly undealt.  The 256^3 D3Q27 fp32 tank (1.81 GB) is even either way
+// (1.157, 1.163 ms per pair), which is where the fp32 line lies.
+uint32_t hydro_deal(const lbm_fields* fl) {
+  const size_t elem = fl->storage == kF32 ? 4 : 2;
+  const size_t bytes = (size_t)fl->Q * fl->d.N * elem;
+  if (bytes < (elem == 4 ? (size_t)1850000000 : (size_t)1000000000)) return kXcdStretch;
+  if (elem == 4) return fl->parity ? 8 : 9;  // 256, 512 blocks
+  return fl->parity ? 8 : 3;
+}
+
 HydroArgs hydro_args(lbm_fields* fl) {
   HydroArgs a{};
   a.d = fl->d;
@@ -462,6 +485,7 @@ HydroArgs hydro_args(lbm_fields* fl) {
   a.F_cur = fl->F_cur;
   a.open = fl->open_face_cells ? 1 : 0;
   a.lin = fl->tiles_linear ? 1 : 0;
+  a.deal = hydro_deal(fl);
   return a;
 }
 
@@ -1950,7 +1974,7 @@ struct lbm_batch {
   void* ring = nullptr;
   uint32_t ring_cap = 0;
   uint32_t* ring_pos = nullptr;
-  uint32_t grid = 0;  // persistent blocks of the collide-stream launch
+  uint32_t grid = 0;  // blocks of the collide-stream launch
   int ncu = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -2090,8 +2114,11 @@ int lbm_batch_create(lbm_ctx* ctx, lbm_fields* const* members, int n, lbm_batch*
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) prop.multiProcessorCount = 256;
     b->ncu = prop.multiProcessorCount;
-    // default: every entry's wave resident at once, capped at 8 blocks per CU
-    b->grid = std::max<uint32_t>(1, std::min<uint32_t>((b->nent + 3) / 4, (uint32_t)b->ncu * 8));
+    // default: a block per four entries.  A resident grid that strides over
+    // the entries (8 blocks per CU) ran 15 tanks of edges 48 to 160 at 0.867
+    // ms per step, this grid at 0.773: the hardware refills a CU wave by wave,
+    // the striding wave waits for its next entry, arguments and loads in turn.
+    b->grid = std::max<uint32_t>(1, (b->nent + 3) / 4);
   }
   for (lbm_fields* fl : b->mem) b->mem_gen.push_back(fl->gen);
   if (rc) {

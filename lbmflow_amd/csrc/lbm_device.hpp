@@ -90,14 +90,21 @@ __device__ __forceinline__ void pop_st(S* plane, uint32_t i, float v) {
   Store<S>::st(plane, i, v);
 }
 
-// Block-id remap: hardware hands consecutive workgroups to the 8 XCDs
-// round-robin; give each XCD a contiguous run of tiles so neighbouring rows
-// share its L2.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n) {
-  constexpr uint32_t X = 8;
-  uint32_t per = n / X, rem = n % X;
-  uint32_t xcd = b % X, local = b / X;
-  return xcd < rem ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
+// Block-id remap: the hardware hands consecutive workgroups to the 8 XCDs
+// round-robin.  kXcdStretch gives each XCD one contiguous stretch of the grid.
+// Any other value deals each run of 8 << deal blocks out so that an XCD gets
+// 1 << deal consecutive blocks of it (0: the plain order; the last, partial
+// run keeps the plain order): blocks that share cache lines meet in one XCD's
+// L2 while all eight XCDs stay in the same part of memory.  Shifts only: the
+// remap runs before a wave's first load.
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n, uint32_t deal) {
+  if (deal == kXcdStretch) {
+    const uint32_t per = n / 8, rem = n % 8, xcd = b % 8, local = b / 8;
+    return xcd < rem ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
+  }
+  const uint32_t run = b >> (deal + 3);
+  if (run == n >> (deal + 3)) return b;
+  return (run << (deal + 3)) + ((b & 7u) << deal) + ((b >> 3) & ((1u << deal) - 1u));
 }
 
 // Wrapped neighbour offsets of one cell (index shift for c = -1 and +1 on

@@ -804,7 +804,7 @@ template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP>
 __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
   // each wave takes one active 64-cell tile; tiles of only solid (or
   // force-listed) cells are never launched
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x, a.deal);
   const uint32_t t = b * 4 + (threadIdx.x >> 6);
   if (t >= a.ntiles) return;
   const uint32_t te = __builtin_amdgcn_readfirstlane(a.tiles[t]);  // one tile per wave
@@ -872,15 +872,17 @@ __global__ __launch_bounds__(256) void k_hydro_list(HydroArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Batched domains: one persistent launch walks the concatenated tile lists
-// of K independent (non-periodic) domains; entry e = (tile, domain).  Each
-// wave strides over entries and reads its tile's domain arguments from the
-// table (wave-uniform, so scalar loads).  Consecutive entries share an XCD.
+// Batched domains: one launch walks the concatenated tile lists of K
+// independent (non-periodic) domains; entry e = (tile, domain).  Each wave
+// strides over entries (a persistent grid, or a grid of one entry per wave)
+// and reads its tile's domain arguments from the table (wave-uniform, so
+// scalar loads).
 // ---------------------------------------------------------------------------
 template <int Q, typename S, int KIND, bool ODD>
 __global__ __launch_bounds__(256) void k_hydro_batch(const HydroArgs* __restrict__ tab,
-                                                     const uint32_t* __restrict__ ent, uint32_t nent) {
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+                                                     const uint32_t* __restrict__ ent, uint32_t nent,
+                                                     uint32_t deal) {
+  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x, deal);
   const uint32_t stride = gridDim.x * 4;
   for (uint32_t e = b * 4 + (threadIdx.x >> 6); e < nent; e += stride) {
     const uint32_t te = __builtin_amdgcn_readfirstlane(ent[2 * (size_t)e]);
@@ -965,10 +967,15 @@ static hipError_t batch_q(int odd, const HydroArgs* tab, const uint32_t* ent, ui
                           const uint32_t* cells, uint32_t ncells, hipStream_t s) {
   if (ent) {
     if (nent == 0) return hipSuccess;
+    // one stretch of entries per XCD for a batch that the last-level cache
+    // holds, the plain order for larger ones (ms per step: 4 tanks of edges 48
+    // to 90, 0.16 GB: 0.0823, 0.0870; 4 of 100 to 160, 0.66 GB: 0.308, 0.295;
+    // 40 tanks, 4.6 GB: 1.830, 1.758)
+    const uint32_t deal = grid < 16384 ? kXcdStretch : 0;
     if (odd)
-      hipLaunchKernelGGL((k_hydro_batch<Q, S, KIND, true>), dim3(grid), dim3(256), 0, s, tab, ent, nent);
+      hipLaunchKernelGGL((k_hydro_batch<Q, S, KIND, true>), dim3(grid), dim3(256), 0, s, tab, ent, nent, deal);
     else
-      hipLaunchKernelGGL((k_hydro_batch<Q, S, KIND, false>), dim3(grid), dim3(256), 0, s, tab, ent, nent);
+      hipLaunchKernelGGL((k_hydro_batch<Q, S, KIND, false>), dim3(grid), dim3(256), 0, s, tab, ent, nent, deal);
   } else {
     if (ncells == 0) return hipSuccess;
     if (odd)

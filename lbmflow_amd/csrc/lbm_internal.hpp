@@ -22,6 +22,9 @@ constexpr uint32_t kTileDeadLo = 1u << 30;
 constexpr uint32_t kTileDeadHi = 1u << 29;
 constexpr uint32_t kTileId = kTileDeadHi - 1u;
 
+// xcd_remap: one contiguous stretch of blocks per XCD
+constexpr uint32_t kXcdStretch = 0xFFFFFFFFu;
+
 enum Storage : int { kF32 = 0, kF16 = 1, kBF16 = 2 };
 
 struct Dom {
@@ -65,6 +68,7 @@ struct HydroArgs {
   float* F_mom;             // N x 3: force of the cached moments
   const float* F_cur;       // N x 3: current field
   int open;                 // fluid on a non-periodic (open) face: wrap every offset
+  uint32_t deal;            // how the tile blocks are dealt to the XCDs (xcd_remap)
   int lin;                  // tiles are 64-cell blocks of the linear index (no axis wraps)
 };
 
