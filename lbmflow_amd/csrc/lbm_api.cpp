@@ -79,6 +79,7 @@ struct lbm_fields {
   // rotating IBM and scalar distributions
   IbmState* ibm = nullptr;
   std::vector<ScalarState*> scalars;
+  std::vector<const void*> g_scalars;  // their current buffers when the step graph was captured
   // device-resident step loop: per-step IBM diagnostics ring, and a HIP
   // graph of two consecutive steps (even + odd) with the key it was
   // captured under (every argument the launches bake in)
@@ -129,6 +130,10 @@ struct lbm_fields {
 // code it is a stand-in, not a device address) but the per-device address
 // that lbm_ctx_create resolves with hipGetSymbolAddress.
 static __device__ __align__(256) float scratch[4 * (size_t)LBM_NOALLOC_MAX_CELLS];
+
+namespace lbm {
+FieldsView view_of(lbm_fields* fl);
+}
 
 namespace {
 
@@ -422,6 +427,8 @@ int count_uncovered(lbm_fields* fl) {
 
 int rebuild_mask(lbm_fields* fl) {
   int rc = normalize_parity(fl);
+  for (ScalarState* sc : fl->scalars)
+    if (!rc) rc = scalar_settle(view_of(fl), sc);
   if (rc) return rc;
   unsigned int* err = nullptr;
   rc = dev_alloc(fl, (void**)&err, sizeof(unsigned int));
@@ -1417,6 +1424,15 @@ static int hydro_step(lbm_fields* fl) {
   return LBM_OK;
 }
 
+// The concentrations of the state a span ends with.
+static int finish_scalars(lbm_fields* fl) {
+  for (ScalarState* sc : fl->scalars) {
+    int rc = scalar_finish(view_of(fl), sc);
+    if (rc) return rc;
+  }
+  return LBM_OK;
+}
+
 int lbm_run_span(lbm_fields* fl, int steps) {
   if (!fl || steps < 0) return LBM_ERR_INVALID;
   int rc = check_steppable(fl);
@@ -1425,7 +1441,7 @@ int lbm_run_span(lbm_fields* fl, int steps) {
     rc = hydro_step(fl);
     if (rc) return rc;
   }
-  return LBM_OK;
+  return finish_scalars(fl);
 }
 
 // The runner's step (runner.rs:1079-1129): clear the force field, rotating
@@ -1474,10 +1490,23 @@ int lbm_run_ibm_span(lbm_fields* fl, int steps, int use_graph, double* torque, l
   // a fill kernel, not a memset, on the stream the graph runs on
   HIPCHK(fl->ctx, launch_fill_f32((float*)fl->ring_pos, 2, 0.0f, s));  // slot, blocks done
   int k = 0;
-  if (use_graph && !fl->timing && steps >= 2) {
+  // a scalar's first steps after a set, a restore or a mask change launch
+  // other kernels than the ones after them: not part of a captured pair
+  auto steady = [&]() {
+    for (ScalarState* sc : fl->scalars)
+      if (!scalar_steady(sc)) return false;
+    return true;
+  };
+  for (; use_graph && k < steps && !steady(); ++k) {
+    rc = ibm_step(fl);
+    if (rc) return rc;
+  }
+  if (use_graph && !fl->timing && steps - k >= 2) {
     const HydroArgs a = hydro_args(fl);
+    std::vector<const void*> scur;
+    for (const ScalarState* sc : fl->scalars) scur.push_back(scalar_current(sc));
     const bool stale = !fl->gexec || fl->g_parity != fl->parity || fl->g_gen != fl->gen ||
-                       fl->g_stash != fl->stash_sel || memcmp(&a, &fl->g_args, sizeof a) != 0;
+                       fl->g_stash != fl->stash_sel || fl->g_scalars != scur || memcmp(&a, &fl->g_args, sizeof a) != 0;
     if (stale) {
       HIPCHK(fl->ctx, drop_graph(s, &fl->gexec, &fl->graph));
       const int parity0 = fl->parity;
@@ -1502,11 +1531,13 @@ int lbm_run_ibm_span(lbm_fields* fl, int steps, int use_graph, double* torque, l
       fl->g_parity = fl->parity;
       fl->g_gen = fl->gen;
       fl->g_stash = fl->stash_sel;
+      fl->g_scalars = scur;
     }
     for (; k + 2 <= steps; k += 2) {
       HIPCHK(fl->ctx, hipGraphLaunch(fl->gexec, s));
       fl->time += 2;
     }
+    for (ScalarState* sc : fl->scalars) scalar_replayed(sc);
     fl->field_present = true;
     fl->field_uniform = false;
   }
@@ -1514,6 +1545,8 @@ int lbm_run_ibm_span(lbm_fields* fl, int steps, int use_graph, double* torque, l
     rc = ibm_step(fl);
     if (rc) return rc;
   }
+  rc = finish_scalars(fl);
+  if (rc) return rc;
   std::vector<lbm_ibm_diag> d(steps);
   rc = ibm_ring_read(view_of(fl), fl->ring, (uint32_t)steps, d.data());
   if (rc) return rc;
@@ -2628,6 +2661,7 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
   }
   if (forward_steps) *forward_steps = advanced;
   ADJ_TRY(snap_restore(fl, fin));
+  ADJ_TRY(finish_scalars(fl));
   ADJ_HIP(hipStreamSynchronize(s));
   reversing = false;
   cleanup();

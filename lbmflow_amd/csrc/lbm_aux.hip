@@ -1,5 +1,4 @@
-// lbm_aux.hip — rotating immersed-boundary direct forcing and the passive
-// scalar advection-diffusion distributions on the device.
+// lbm_aux.hip — rotating immersed-boundary direct forcing on the device.
 //
 // IBM (Solver::apply_rotating_ibm, solver.rs:3016-3282, rotating_ibm.rs):
 // marker positions are frozen, as in the reference, so the marker stencils
@@ -13,12 +12,6 @@
 // per-cell spread; fixed-tree marker reductions), commits the force field
 // and records the diagnostics.  The slip-tolerance early exit is taken
 // inside that block, so the host never waits inside a sweep.
-//
-// Scalar ADE: BGK collide toward h_eq = w C (1 + c.u/cs^2) with the cached
-// concentration and the post-step hydro velocity, pull streaming with
-// half-way bounce-back at solids, C = sum h (solver.rs:2113-2205,
-// scalar.rs:6-15).  The hydro lattice (reference) and D3Q7 (cs^2 = 1/4) are
-// both supported.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -31,15 +24,6 @@ namespace lbm {
 namespace {
 
 inline uint32_t nblk(size_t n, uint32_t bs = 256) { return (uint32_t)((n + bs - 1) / bs); }
-
-#define AUXCHK(v, expr)                                                      \
-  do {                                                                       \
-    hipError_t _e = (expr);                                                  \
-    if (_e != hipSuccess) {                                                  \
-      if ((v).ctx_err) *(v).ctx_err = std::string(#expr ": ") + hipGetErrorString(_e); \
-      return LBM_ERR_DEVICE;                                                 \
-    }                                                                        \
-  } while (0)
 
 }  // namespace
 
@@ -1518,295 +1502,6 @@ int ibm_ring_read(const FieldsView& v, const void* ring, uint32_t n, lbm_ibm_dia
   }
   for (uint32_t k = 0; k < n; ++k) diag_to_abi(h[k], out + k);
   return LBM_OK;
-}
-
-// ===========================================================================
-// passive scalar ADE
-// ===========================================================================
-struct ScalarState {
-  int Qs = 7;
-  double D = 0.0;
-  float omega = 1.0f;
-  float* h = nullptr;
-  float* h2 = nullptr;
-  float* C = nullptr;
-  float* mom = nullptr;  // rho, ux, uy, uz (4 x N)
-  double* partials = nullptr;
-  uint32_t npartials = 1024;
-};
-
-// h_eq of scalar_equilibrium (scalar.rs:6-15) for the hydro lattice; the
-// D3Q7 form uses 1/cs^2 = 4.
-template <int Qs, int q>
-__device__ __forceinline__ float heq_q(float conc, float ux, float uy, float uz) {
-  const float cu = cdot<q>(ux, uy, uz);
-  constexpr float k = Qs == 7 ? 4.0f : 3.0f;
-  return lat_wf(Qs, q) * conc * (1.0f + k * cu);
-}
-
-template <int Qs>
-__global__ void k_scalar_set(Dom d, const float* conc, const float* mom, float* h, float* C) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N) return;
-  const float c = conc[i];
-  const float ux = mom[d.N + i], uy = mom[2 * (size_t)d.N + i], uz = mom[3 * (size_t)d.N + i];
-  C[i] = c;
-  sfor<0, Qs>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    h[(size_t)q * d.N + i] = heq_q<Qs, q>(c, ux, uy, uz);
-  });
-}
-
-template <int Qs>
-__global__ void k_scalar_collide(Dom d, const uint32_t* mask, float* h, const float* C, const float* mom,
-                                 float omega) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N || (mask[i] & kMaskSolid)) return;
-  const float c = C[i];
-  const float ux = mom[d.N + i], uy = mom[2 * (size_t)d.N + i], uz = mom[3 * (size_t)d.N + i];
-  sfor<0, Qs>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    float* p = h + (size_t)q * d.N + i;
-    const float hq = *p;
-    *p = hq - omega * (hq - heq_q<Qs, q>(c, ux, uy, uz));
-  });
-}
-
-template <int Qs>
-__global__ void k_scalar_stream(Dom d, const uint32_t* mask, const float* h, float* h2, float* C) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N) return;
-  const uint32_t m = mask[i];
-  if (m & kMaskSolid) {
-    C[i] = 0.0f;
-    sfor<0, Qs>([&](auto qc) { h2[(size_t)decltype(qc)::value * d.N + i] = 0.0f; });
-    return;
-  }
-  uint32_t x, y, z;
-  cell_xyz(d, i, x, y, z);
-  const Nbr nb(d, x, y, z);
-  float sum = 0.0f;
-  sfor<0, Qs>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    constexpr int o = lat_opp(q);
-    float v;
-    if ((m >> q) & 1u) {  // source i - c_q is solid: bounce back own h_opp
-      v = h[(size_t)o * d.N + i];
-    } else {
-      const uint32_t s = i + (uint32_t)nb.template off<-lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>();
-      v = h[(size_t)q * d.N + s];
-    }
-    h2[(size_t)q * d.N + i] = v;
-    sum = sum + v;
-  });
-  C[i] = sum;
-}
-
-// Two-pass CV over fluid cells (qoi::scalar_cv, qoi.rs:507-532), for the
-// whole fluid (parts = 1) or the three compartments of compartment_cv
-// (qoi.rs:699-739, parts = 3): a fluid cell of plane z is "top" when
-// (z + 0.5)/nz >= 2/3, else "near_impeller" when an impeller height is given
-// and |(z + 0.5) - z_imp| <= nz/6, else "bulk" (f64, the reference's
-// expressions).  Pass 0 sums counts and values per compartment, pass 1 the
-// squared deviations from the compartment means.  Per block: 6 doubles
-// (count, sum per compartment; pass 1 fills the first 3 with the variances).
-__global__ __launch_bounds__(256) void k_cv_pass(Dom d, const uint32_t* mask, const float* C, int pass, int parts,
-                                                 int has_imp, double imp_z, double m0, double m1, double m2,
-                                                 double* partials) {
-  __shared__ double lds[4 * 6];
-  double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  const double nz = (double)d.nz;
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < d.N; i += gridDim.x * 256) {
-    if (mask[i] & kMaskSolid) continue;
-    int k = 0;
-    if (parts == 3) {
-      const double zc = (double)(i / (d.nx * d.ny)) + 0.5;
-      if (zc / nz >= 2.0 / 3.0)
-        k = 0;
-      else if (has_imp && fabs(zc - imp_z) <= nz / 6.0)
-        k = 2;
-      else
-        k = 1;
-    }
-    const double v = (double)C[i];
-    if (pass == 0) {
-      acc[2 * k] += 1.0;
-      acc[2 * k + 1] += v;
-    } else {
-      const double dv = v - (k == 0 ? m0 : (k == 1 ? m1 : m2));
-      acc[k] += dv * dv;
-    }
-  }
-  block_sum256<6>(acc, lds);
-  if (threadIdx.x == 0)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) partials[6 * blockIdx.x + k] = acc[k];
-}
-
-ScalarState* scalar_create(const FieldsView& v, double diffusivity, int Qs, std::string* err) {
-  ScalarState* s = new ScalarState();
-  s->Qs = Qs;
-  s->D = diffusivity;
-  // omega = T(1/(3D + 1/2)) on the hydro lattice (solver.rs:2131);
-  // D3Q7 maps tau = D/cs^2 + 1/2 = 4D + 1/2.
-  s->omega = Qs == 7 ? (float)(1.0 / (4.0 * diffusivity + 0.5)) : (float)(1.0 / (3.0 * diffusivity + 0.5));
-  const size_t N = v.d.N;
-  hipError_t e = hipMalloc((void**)&s->h, (size_t)Qs * N * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->h2, (size_t)Qs * N * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->C, N * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->mom, 4 * N * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->partials, 6 * s->npartials * sizeof(double));
-  if (e == hipSuccess) e = hipMemsetAsync(s->h, 0, (size_t)Qs * N * 4, v.stream);
-  if (e == hipSuccess) e = hipMemsetAsync(s->h2, 0, (size_t)Qs * N * 4, v.stream);
-  if (e == hipSuccess) e = hipMemsetAsync(s->C, 0, N * 4, v.stream);
-  if (e != hipSuccess) {
-    *err = std::string("scalar allocation failed: ") + hipGetErrorString(e);
-    scalar_destroy(s);
-    return nullptr;
-  }
-  return s;
-}
-
-void scalar_destroy(ScalarState* s) {
-  if (!s) return;
-  for (void* p : {(void*)s->h, (void*)s->h2, (void*)s->C, (void*)s->mom, (void*)s->partials})
-    if (p) (void)hipFree(p);
-  delete s;
-}
-
-static int refresh_mom(const FieldsView& v, ScalarState* s) {
-  const size_t N = v.d.N;
-  AUXCHK(v, launch_moments(v.Q, v.storage, v.parity, v.d, v.f, v.mask, v.F_mom, v.hp, s->mom, s->mom + N,
-                           s->mom + 2 * N, s->mom + 3 * N, v.stream));
-  return LBM_OK;
-}
-
-int scalar_set(const FieldsView& v, ScalarState* s, const float* conc) {
-  const size_t N = v.d.N;
-  float* dc = nullptr;
-  AUXCHK(v, hipMalloc((void**)&dc, N * 4));
-  AUXCHK(v, hipMemcpyAsync(dc, conc, N * 4, hipMemcpyHostToDevice, v.stream));
-  int rc = refresh_mom(v, s);
-  if (rc) return rc;
-  if (s->Qs == 7)
-    hipLaunchKernelGGL((k_scalar_set<7>), dim3(nblk(N)), dim3(256), 0, v.stream, v.d, dc, s->mom, s->h, s->C);
-  else if (s->Qs == 19)
-    hipLaunchKernelGGL((k_scalar_set<19>), dim3(nblk(N)), dim3(256), 0, v.stream, v.d, dc, s->mom, s->h, s->C);
-  else
-    hipLaunchKernelGGL((k_scalar_set<27>), dim3(nblk(N)), dim3(256), 0, v.stream, v.d, dc, s->mom, s->h, s->C);
-  AUXCHK(v, hipGetLastError());
-  AUXCHK(v, hipStreamSynchronize(v.stream));
-  (void)hipFree(dc);
-  return LBM_OK;
-}
-
-// checkpoint access: the distribution h (current), its ping-pong partner h2
-// (after a step: the post-collision populations), the concentration, and
-// the lattice size and diffusivity
-int scalar_info(const ScalarState* s, int* Qs, double* D) {
-  *Qs = s->Qs;
-  *D = s->D;
-  return LBM_OK;
-}
-
-int scalar_get_state(const FieldsView& v, ScalarState* s, float* h, float* h2, float* C) {
-  const size_t N = v.d.N, bytes = (size_t)s->Qs * N * 4;
-  AUXCHK(v, hipMemcpyAsync(h, s->h, bytes, hipMemcpyDeviceToHost, v.stream));
-  AUXCHK(v, hipMemcpyAsync(h2, s->h2, bytes, hipMemcpyDeviceToHost, v.stream));
-  AUXCHK(v, hipMemcpyAsync(C, s->C, N * 4, hipMemcpyDeviceToHost, v.stream));
-  AUXCHK(v, hipStreamSynchronize(v.stream));
-  return LBM_OK;
-}
-
-int scalar_put_state(const FieldsView& v, ScalarState* s, const float* h, const float* h2, const float* C) {
-  const size_t N = v.d.N, bytes = (size_t)s->Qs * N * 4;
-  AUXCHK(v, hipMemcpyAsync(s->h, h, bytes, hipMemcpyHostToDevice, v.stream));
-  AUXCHK(v, hipMemcpyAsync(s->h2, h2, bytes, hipMemcpyHostToDevice, v.stream));
-  AUXCHK(v, hipMemcpyAsync(s->C, C, N * 4, hipMemcpyHostToDevice, v.stream));
-  AUXCHK(v, hipStreamSynchronize(v.stream));
-  return LBM_OK;
-}
-
-int scalar_gather(const FieldsView& v, ScalarState* s, float* conc) {
-  AUXCHK(v, hipMemcpyAsync(conc, s->C, (size_t)v.d.N * 4, hipMemcpyDeviceToHost, v.stream));
-  AUXCHK(v, hipStreamSynchronize(v.stream));
-  return LBM_OK;
-}
-
-template <int Qs>
-static void scalar_step_q(const FieldsView& v, ScalarState* s) {
-  const uint32_t g = nblk(v.d.N);
-  hipLaunchKernelGGL((k_scalar_collide<Qs>), dim3(g), dim3(256), 0, v.stream, v.d, v.mask, s->h, s->C, s->mom,
-                     s->omega);
-  hipLaunchKernelGGL((k_scalar_stream<Qs>), dim3(g), dim3(256), 0, v.stream, v.d, v.mask, s->h, s->h2, s->C);
-}
-
-int scalar_step(const FieldsView& v, ScalarState* s) {
-  int rc = refresh_mom(v, s);
-  if (rc) return rc;
-  if (s->Qs == 7)
-    scalar_step_q<7>(v, s);
-  else if (s->Qs == 19)
-    scalar_step_q<19>(v, s);
-  else
-    scalar_step_q<27>(v, s);
-  AUXCHK(v, hipGetLastError());
-  std::swap(s->h, s->h2);
-  return LBM_OK;
-}
-
-// Both passes of k_cv_pass; results per compartment (parts = 1 or 3).
-static int cv_parts(const FieldsView& v, ScalarState* s, int parts, int has_imp, double imp_z, double* cv,
-                    int* defined, int64_t* counts) {
-  const uint32_t np = std::min<uint32_t>(s->npartials, nblk(v.d.N));
-  std::vector<double> h(6 * (size_t)np);
-  auto run = [&](int pass, const double* mean) -> int {
-    hipLaunchKernelGGL(k_cv_pass, dim3(np), dim3(256), 0, v.stream, v.d, v.mask, s->C, pass, parts, has_imp, imp_z,
-                       mean[0], mean[1], mean[2], s->partials);
-    AUXCHK(v, hipGetLastError());
-    AUXCHK(v, hipMemcpyAsync(h.data(), s->partials, h.size() * sizeof(double), hipMemcpyDeviceToHost, v.stream));
-    AUXCHK(v, hipStreamSynchronize(v.stream));
-    return LBM_OK;
-  };
-  const double zero[3] = {0.0, 0.0, 0.0};
-  int rc = run(0, zero);
-  if (rc) return rc;
-  double n[3] = {0, 0, 0}, sum[3] = {0, 0, 0}, mean[3] = {0, 0, 0};
-  for (uint32_t b = 0; b < np; ++b)
-    for (int k = 0; k < parts; ++k) {
-      n[k] += h[6 * (size_t)b + 2 * k];
-      sum[k] += h[6 * (size_t)b + 2 * k + 1];
-    }
-  bool any = false;
-  for (int k = 0; k < parts; ++k) {
-    counts[k] = (int64_t)n[k];
-    defined[k] = 0;
-    cv[k] = 0.0;
-    if (n[k] == 0.0) continue;
-    mean[k] = sum[k] / n[k];
-    if (mean[k] == 0.0) continue;
-    defined[k] = 1;
-    any = true;
-  }
-  if (!any) return LBM_OK;
-  rc = run(1, mean);
-  if (rc) return rc;
-  double var[3] = {0, 0, 0};
-  for (uint32_t b = 0; b < np; ++b)
-    for (int k = 0; k < parts; ++k) var[k] += h[6 * (size_t)b + k];
-  for (int k = 0; k < parts; ++k)
-    if (defined[k]) cv[k] = std::sqrt(var[k] / n[k]) / std::fabs(mean[k]);
-  return LBM_OK;
-}
-
-int scalar_cv(const FieldsView& v, ScalarState* s, double* cv, int* defined) {
-  int64_t count = 0;
-  return cv_parts(v, s, 1, 0, 0.0, cv, defined, &count);
-}
-
-int scalar_compartment_cv(const FieldsView& v, ScalarState* s, int has_imp, double imp_z, double cv[3],
-                          int defined[3], int64_t counts[3]) {
-  return cv_parts(v, s, 3, has_imp, imp_z, cv, defined, counts);
 }
 
 }  // namespace lbm

@@ -1,5 +1,5 @@
 // lbm_aux.hpp — host interface of the rotating-IBM and scalar-ADE device
-// paths (lbm_aux.hip), used by the C-ABI layer.  Not part of the public ABI.
+// paths (lbm_aux.hip, lbm_scalar.hip), used by the C-ABI layer.  Not part of the public ABI.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -10,6 +10,15 @@
 #include "lbm_internal.hpp"
 
 namespace lbm {
+
+#define AUXCHK(v, expr)                                                      \
+  do {                                                                       \
+    hipError_t _e = (expr);                                                  \
+    if (_e != hipSuccess) {                                                  \
+      if ((v).ctx_err) *(v).ctx_err = std::string(#expr ": ") + hipGetErrorString(_e); \
+      return LBM_ERR_DEVICE;                                                 \
+    }                                                                        \
+  } while (0)
 
 // The slice of a domain's state the auxiliary paths need.
 struct FieldsView {
@@ -79,12 +88,24 @@ int ibm_adjoint(const FieldsView& v, IbmState* s, const double* Fbar, const doub
 // n ring records (entry-major, instance-minor) to ABI diagnostics
 int ibm_ring_read(const FieldsView& v, const void* ring, uint32_t n, lbm_ibm_diag* out);
 
-// Passive scalar ADE (Solver::step_scalar_distributions, solver.rs:2113-2205).
+// Passive scalar ADE (Solver::step_scalar_distributions, solver.rs:2113-2205;
+// lbm_scalar.hip).  scalar_step leaves the concentration to scalar_finish,
+// which every call that steps a scalar ends with; scalar_settle puts both
+// buffers into the reference's form before the masks change.
 ScalarState* scalar_create(const FieldsView& v, double diffusivity, int Qs, std::string* err);
 void scalar_destroy(ScalarState* s);
 int scalar_set(const FieldsView& v, ScalarState* s, const float* conc);
 int scalar_gather(const FieldsView& v, ScalarState* s, float* conc);
 int scalar_step(const FieldsView& v, ScalarState* s);
+int scalar_finish(const FieldsView& v, ScalarState* s);
+int scalar_settle(const FieldsView& v, ScalarState* s);
+// whether a step launches the same kernels as the next one (false right
+// after the concentration, the state or the masks were set)
+bool scalar_steady(const ScalarState* s);
+// the buffer the next step reads (a captured pair of steps is bound to it),
+// and the mark that captured steps ran
+const void* scalar_current(const ScalarState* s);
+void scalar_replayed(ScalarState* s);
 int scalar_cv(const FieldsView& v, ScalarState* s, double* cv, int* defined);
 int scalar_info(const ScalarState* s, int* Qs, double* D);
 int scalar_get_state(const FieldsView& v, ScalarState* s, float* h, float* h2, float* C);

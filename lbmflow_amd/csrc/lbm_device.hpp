@@ -122,6 +122,9 @@ struct Nbr {
     zm = (z == 0 ? (int32_t)d.nz - 1 : -1) * nxy;
     zp = (z == d.nz - 1 ? -((int32_t)d.nz - 1) : 1) * nxy;
   }
+  // no axis wraps: the same shifts for every cell
+  __device__ __forceinline__ explicit Nbr(const Dom& d)
+      : xm(-1), xp(1), ym(-(int32_t)d.nx), yp((int32_t)d.nx), zm(-(int32_t)(d.nx * d.ny)), zp((int32_t)(d.nx * d.ny)) {}
   template <int cx, int cy, int cz>
   __device__ __forceinline__ int32_t off() const {
     int32_t o = 0;
