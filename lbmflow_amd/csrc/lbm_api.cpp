@@ -30,6 +30,7 @@ struct lbm_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
+  Readback rb;
 };
 
 struct lbm_fields {
@@ -367,8 +368,8 @@ static int normalize_parity(lbm_fields* fl) {
   int rc = dev_alloc(fl, (void**)&tmp, bytes);
   if (rc) return rc;
   hipStream_t s = fl->ctx->stream;
-  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 1, 1, fl->d, fl->f, tmp, fl->mask, s));
-  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 0, 0, fl->d, fl->f, tmp, fl->mask, s));
+  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 1, 1, fl->d, fl->f, tmp, fl->mask, 0, fl->d.N, s));
+  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 0, 0, fl->d, fl->f, tmp, fl->mask, 0, fl->d.N, s));
   HIPCHK(fl->ctx, hipStreamSynchronize(s));
   dev_free(fl, tmp, bytes);
   fl->parity = 0;
@@ -496,6 +497,16 @@ HydroArgs hydro_args(lbm_fields* fl) {
   return a;
 }
 
+// one device array to caller memory
+int read_array(lbm_fields* fl, void* dst, const void* src, size_t bytes) {
+  const hipError_t read_back = fl->ctx->rb.read(fl->ctx->device, fl->ctx->stream, 1, [&](int, std::vector<Readback::Seg>& segs) {
+    segs.push_back({dst, src, bytes});
+    return hipSuccess;
+  });
+  HIPCHK(fl->ctx, read_back);
+  return LBM_OK;
+}
+
 // Cached moments now carry the current field (Backend::update_moments).
 int refresh_moments(lbm_fields* fl) {
   if (fl->F_mom && !fl->flist_host.empty())
@@ -512,6 +523,8 @@ FieldsView view_of(lbm_fields* fl) {
   FieldsView v{};
   v.ctx_err = &fl->ctx->err;
   v.stream = fl->ctx->stream;
+  v.device = fl->ctx->device;
+  v.rb = &fl->ctx->rb;
   v.Q = fl->Q;
   v.storage = fl->storage;
   v.d = fl->d;
@@ -835,7 +848,7 @@ int lbm_stage_in(lbm_fields* fl, const float* f) {
   if (rc) return rc;
   hipStream_t s = fl->ctx->stream;
   HIPCHK(fl->ctx, hipMemcpyAsync(tmp, f, bytes, hipMemcpyHostToDevice, s));
-  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 0, 0, fl->d, fl->f, tmp, fl->mask, s));
+  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 0, 0, fl->d, fl->f, tmp, fl->mask, 0, fl->d.N, s));
   HIPCHK(fl->ctx, hipStreamSynchronize(s));
   dev_free(fl, tmp, bytes);
   fl->parity = 0;
@@ -844,15 +857,21 @@ int lbm_stage_in(lbm_fields* fl, const float* f) {
 
 int lbm_stage_out(lbm_fields* fl, float* f) {
   if (!fl || !f) return LBM_ERR_INVALID;
-  const size_t bytes = (size_t)fl->Q * fl->d.N * 4;
-  float* tmp = nullptr;
-  int rc = dev_alloc(fl, (void**)&tmp, bytes);
-  if (rc) return rc;
   hipStream_t s = fl->ctx->stream;
-  HIPCHK(fl->ctx, launch_stage(fl->Q, fl->storage, 1, fl->parity, fl->d, fl->f, tmp, fl->mask, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(f, tmp, bytes, hipMemcpyDeviceToHost, s));
-  HIPCHK(fl->ctx, hipStreamSynchronize(s));
-  dev_free(fl, tmp, bytes);
+  Readback& rb = fl->ctx->rb;
+  float* w = (float*)rb.work();
+  if (!w) return fail(fl->ctx, LBM_ERR_NOMEM, "read-back workspace of %zu bytes", Readback::kWorkBytes);
+  // pieces of as many cells as the workspace holds Q planes of
+  const uint32_t N = fl->d.N, Q = (uint32_t)fl->Q;
+  const uint32_t per = (uint32_t)(Readback::kWorkBytes / 4 / Q) / 1024 * 1024;
+  const int pieces = (int)((N + per - 1) / per);
+  const hipError_t read_back = rb.read(fl->ctx->device, s, pieces, [&](int p, std::vector<Readback::Seg>& segs) {
+    const uint32_t i0 = (uint32_t)p * per, cnt = std::min(per, N - i0);
+    for (uint32_t q = 0; q < Q; ++q)
+      segs.push_back({f + (size_t)q * N + i0, w + (size_t)q * cnt, (size_t)cnt * 4});
+    return launch_stage(fl->Q, fl->storage, 1, fl->parity, fl->d, fl->f, w, fl->mask, i0, cnt, s);
+  });
+  HIPCHK(fl->ctx, read_back);
   return LBM_OK;
 }
 
@@ -926,9 +945,7 @@ int lbm_read_force_field(lbm_fields* fl, float* ff, int* present) {
     std::fill(ff, ff + N3(fl), 0.0f);
     return LBM_OK;
   }
-  HIPCHK(fl->ctx, hipMemcpyAsync(ff, fl->F_cur, N3(fl) * 4, hipMemcpyDeviceToHost, fl->ctx->stream));
-  HIPCHK(fl->ctx, hipStreamSynchronize(fl->ctx->stream));
-  return LBM_OK;
+  return read_array(fl, ff, fl->F_cur, N3(fl) * 4);
 }
 
 // ---- WALE LES ------------------------------------------------------------
@@ -1025,9 +1042,7 @@ int lbm_gather_omega_field(lbm_fields* fl, float* omega, int* present) {
   if (!fl || !omega || !present) return LBM_ERR_INVALID;
   *present = fl->omega ? 1 : 0;
   if (!fl->omega) return LBM_OK;
-  HIPCHK(fl->ctx, hipMemcpyAsync(omega, fl->omega, (size_t)fl->d.N * 4, hipMemcpyDeviceToHost, fl->ctx->stream));
-  HIPCHK(fl->ctx, hipStreamSynchronize(fl->ctx->stream));
-  return LBM_OK;
+  return read_array(fl, omega, fl->omega, (size_t)fl->d.N * 4);
 }
 
 int lbm_set_wale(lbm_fields* fl, int enabled, double cw, double tau_eff_max) {
@@ -1592,19 +1607,21 @@ int64_t lbm_time(const lbm_fields* fl) { return fl ? fl->time : -1; }
 
 int lbm_read_moments(lbm_fields* fl, float* rho, float* ux, float* uy, float* uz) {
   if (!fl || !rho || !ux || !uy || !uz) return LBM_ERR_INVALID;
-  const size_t n = fl->d.N;
-  float* buf = nullptr;
-  int rc = dev_alloc(fl, (void**)&buf, 4 * n * 4);
-  if (rc) return rc;
   hipStream_t s = fl->ctx->stream;
-  HIPCHK(fl->ctx, launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, buf,
-                                 buf + n, buf + 2 * n, buf + 3 * n, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(rho, buf, n * 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(ux, buf + n, n * 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(uy, buf + 2 * n, n * 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(uz, buf + 3 * n, n * 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(fl->ctx, hipStreamSynchronize(s));
-  dev_free(fl, buf, 4 * n * 4);
+  Readback& rb = fl->ctx->rb;
+  float* w = (float*)rb.work();
+  if (!w) return fail(fl->ctx, LBM_ERR_NOMEM, "read-back workspace of %zu bytes", Readback::kWorkBytes);
+  const uint32_t N = fl->d.N;
+  const uint32_t per = (uint32_t)(Readback::kWorkBytes / 16);
+  const int pieces = (int)((N + per - 1) / per);
+  float* const out[4] = {rho, ux, uy, uz};
+  const hipError_t read_back = rb.read(fl->ctx->device, s, pieces, [&](int p, std::vector<Readback::Seg>& segs) {
+    const uint32_t i0 = (uint32_t)p * per, cnt = std::min(per, N - i0);
+    for (int k = 0; k < 4; ++k) segs.push_back({out[k] + i0, w + (size_t)k * cnt, (size_t)cnt * 4});
+    return launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, i0, cnt, w,
+                          w + cnt, w + 2 * (size_t)cnt, w + 3 * (size_t)cnt, s);
+  });
+  HIPCHK(fl->ctx, read_back);
   return LBM_OK;
 }
 
@@ -1620,8 +1637,8 @@ int lbm_read_moments_noalloc(lbm_fields* fl, float* rho, float* ux, float* uy, f
     return fail(fl->ctx, LBM_ERR_DEVICE, "lbm_read_moments_noalloc: no staging address for device %d: %s",
                 fl->ctx->device, hipGetErrorString(se));
   hipStream_t s = fl->ctx->stream;
-  HIPCHK(fl->ctx, launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, buf,
-                                 buf + n, buf + 2 * n, buf + 3 * n, s));
+  HIPCHK(fl->ctx, launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, 0,
+                                 (uint32_t)n, buf, buf + n, buf + 2 * n, buf + 3 * n, s));
   HIPCHK(fl->ctx, hipMemcpyAsync(rho, buf, n * 4, hipMemcpyDeviceToHost, s));
   HIPCHK(fl->ctx, hipMemcpyAsync(ux, buf + n, n * 4, hipMemcpyDeviceToHost, s));
   HIPCHK(fl->ctx, hipMemcpyAsync(uy, buf + 2 * n, n * 4, hipMemcpyDeviceToHost, s));

@@ -8,6 +8,7 @@
 
 #include "../../include/lbm_hip.h"
 #include "lbm_internal.hpp"
+#include "lbm_readback.hpp"
 
 namespace lbm {
 
@@ -24,6 +25,8 @@ namespace lbm {
 struct FieldsView {
   std::string* ctx_err;
   hipStream_t stream;
+  int device;
+  Readback* rb;
   int Q, storage;
   Dom d;
   void* f;

@@ -216,16 +216,17 @@ hipError_t launch_build_mask(int Q, const Dom& d, const uint8_t* solid, const fl
                              unsigned int* err_count, hipStream_t s);
 hipError_t launch_mark_forced(const uint32_t* flist, uint32_t n, uint32_t* mask, hipStream_t s);
 hipError_t launch_tile_flags(const Dom& d, const uint32_t* mask, uint8_t* flags, int linear, hipStream_t s);
+// cells i0 .. i0 + cnt - 1 (host_layout: Q planes of cnt)
 hipError_t launch_stage(int Q, int storage, int dir, int odd, const Dom& d, void* f, float* host_layout,
-                        const uint32_t* mask, hipStream_t s);
+                        const uint32_t* mask, uint32_t i0, uint32_t cnt, hipStream_t s);
 hipError_t launch_init_with(int Q, int storage, const Dom& d, void* f, const uint32_t* mask, const float* rho,
                             const float* u, float tau, hipStream_t s);
 // previous step's post-collision populations (compact Q x N), see k_poststate
 hipError_t launch_poststate(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
                             const float* wall_u, float* out, hipStream_t s);
 hipError_t launch_moments(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
-                          const float* F_mom, HydroParams p, float* rho, float* ux, float* uy, float* uz,
-                          hipStream_t s);
+                          const float* F_mom, HydroParams p, uint32_t i0, uint32_t cnt, float* rho, float* ux,
+                          float* uy, float* uz, hipStream_t s);
 hipError_t launch_reduce(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
                          const float* F_mom, HydroParams p, int kind, int axis, double* partials,
                          uint32_t npartials, hipStream_t s);

@@ -26,13 +26,15 @@ __global__ void k_clear_batch(const HydroArgs* __restrict__ tab, const uint32_t*
 // moments readback (moments_row with the cached-moment force F_u + F_mom)
 template <int Q, typename S>
 __global__ void k_moments(Dom d, const S* f, const uint32_t* mask, const float* F_mom, HydroParams p, int odd,
-                          float* rho, float* ux, float* uy, float* uz) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N) return;
+                          uint32_t i0, uint32_t cnt, float* rho, float* ux, float* uy, float* uz) {
+  // cells i0 .. i0 + cnt - 1, written at 0 .. cnt - 1
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= cnt) return;
+  const uint32_t i = i0 + k;
   const uint32_t m = mask[i];
   if (m & kMaskSolid) {
-    rho[i] = 1.0f;
-    ux[i] = uy[i] = uz[i] = 0.0f;
+    rho[k] = 1.0f;
+    ux[k] = uy[k] = uz[k] = 0.0f;
     return;
   }
   uint32_t x, y, z;
@@ -52,22 +54,24 @@ __global__ void k_moments(Dom d, const S* f, const uint32_t* mask, const float* 
   }
   float r, a, b, c;
   moments<Q>(fv, Fm, fon, r, a, b, c);
-  rho[i] = r;
-  ux[i] = a;
-  uy[i] = b;
-  uz[i] = c;
+  rho[k] = r;
+  ux[k] = a;
+  uy[k] = b;
+  uz[k] = c;
 }
 
 // stage in (dir 0: host layout -> device, parity reset to even) /
 // stage out (dir 1: device -> host layout, de-permuted by parity).
+// Cells i0 .. i0 + cnt - 1; the host layout holds Q planes of cnt.
 template <int Q, typename S>
-__global__ void k_stage(Dom d, S* f, float* h, const uint32_t* mask, int dir, int odd) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.N) return;
+__global__ void k_stage(Dom d, S* f, float* h, const uint32_t* mask, int dir, int odd, uint32_t i0, uint32_t cnt) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= cnt) return;
+  const uint32_t i = i0 + k;
   if (dir == 0) {
     sfor<0, Q>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
-      pop_st<S, Q, q>(f + (size_t)q * d.ps, i, h[(size_t)q * d.N + i]);
+      pop_st<S, Q, q>(f + (size_t)q * d.ps, i, h[(size_t)q * cnt + k]);
     });
     return;
   }
@@ -78,7 +82,7 @@ __global__ void k_stage(Dom d, S* f, float* h, const uint32_t* mask, int dir, in
   const Nbr nb(d, x, y, z);
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    h[(size_t)q * d.N + i] = solid ? 0.0f : read_pop<Q, S, q>(f, d.ps, nb, i, m, odd != 0);
+    h[(size_t)q * cnt + k] = solid ? 0.0f : read_pop<Q, S, q>(f, d.ps, nb, i, m, odd != 0);
   });
 }
 
@@ -546,20 +550,20 @@ hipError_t launch_mark_forced(const uint32_t* flist, uint32_t n, uint32_t* mask,
 }
 
 template <typename S>
-static hipError_t stage_s(int Q, int dir, int odd, const Dom& d, void* f, float* h, const uint32_t* mask,
-                          hipStream_t s) {
+static hipError_t stage_s(int Q, int dir, int odd, const Dom& d, void* f, float* h, const uint32_t* mask, uint32_t i0,
+                          uint32_t cnt, hipStream_t s) {
   if (Q == 19)
-    hipLaunchKernelGGL((k_stage<19, S>), dim3(blocks_for(d.N)), dim3(256), 0, s, d, (S*)f, h, mask, dir, odd);
+    hipLaunchKernelGGL((k_stage<19, S>), dim3(blocks_for(cnt)), dim3(256), 0, s, d, (S*)f, h, mask, dir, odd, i0, cnt);
   else
-    hipLaunchKernelGGL((k_stage<27, S>), dim3(blocks_for(d.N)), dim3(256), 0, s, d, (S*)f, h, mask, dir, odd);
+    hipLaunchKernelGGL((k_stage<27, S>), dim3(blocks_for(cnt)), dim3(256), 0, s, d, (S*)f, h, mask, dir, odd, i0, cnt);
   return hipGetLastError();
 }
 
 hipError_t launch_stage(int Q, int storage, int dir, int odd, const Dom& d, void* f, float* h, const uint32_t* mask,
-                        hipStream_t s) {
-  if (storage == kF32) return stage_s<float>(Q, dir, odd, d, f, h, mask, s);
-  if (storage == kF16) return stage_s<_Float16>(Q, dir, odd, d, f, h, mask, s);
-  return stage_s<bf16s>(Q, dir, odd, d, f, h, mask, s);
+                        uint32_t i0, uint32_t cnt, hipStream_t s) {
+  if (storage == kF32) return stage_s<float>(Q, dir, odd, d, f, h, mask, i0, cnt, s);
+  if (storage == kF16) return stage_s<_Float16>(Q, dir, odd, d, f, h, mask, i0, cnt, s);
+  return stage_s<bf16s>(Q, dir, odd, d, f, h, mask, i0, cnt, s);
 }
 
 template <typename S>
@@ -581,13 +585,14 @@ hipError_t launch_init_with(int Q, int storage, const Dom& d, void* f, const uin
 
 template <typename S>
 static hipError_t moments_s(int Q, int odd, const Dom& d, const void* f, const uint32_t* mask, const float* F_mom,
-                            HydroParams p, float* rho, float* ux, float* uy, float* uz, hipStream_t s) {
+                            HydroParams p, uint32_t i0, uint32_t cnt, float* rho, float* ux, float* uy, float* uz,
+                            hipStream_t s) {
   if (Q == 19)
-    hipLaunchKernelGGL((k_moments<19, S>), dim3(blocks_for(d.N)), dim3(256), 0, s, d, (const S*)f, mask, F_mom, p,
-                       odd, rho, ux, uy, uz);
+    hipLaunchKernelGGL((k_moments<19, S>), dim3(blocks_for(cnt)), dim3(256), 0, s, d, (const S*)f, mask, F_mom, p,
+                       odd, i0, cnt, rho, ux, uy, uz);
   else
-    hipLaunchKernelGGL((k_moments<27, S>), dim3(blocks_for(d.N)), dim3(256), 0, s, d, (const S*)f, mask, F_mom, p,
-                       odd, rho, ux, uy, uz);
+    hipLaunchKernelGGL((k_moments<27, S>), dim3(blocks_for(cnt)), dim3(256), 0, s, d, (const S*)f, mask, F_mom, p,
+                       odd, i0, cnt, rho, ux, uy, uz);
   return hipGetLastError();
 }
 
@@ -611,11 +616,11 @@ hipError_t launch_poststate(int Q, int storage, int odd, const Dom& d, const voi
 }
 
 hipError_t launch_moments(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
-                          const float* F_mom, HydroParams p, float* rho, float* ux, float* uy, float* uz,
-                          hipStream_t s) {
-  if (storage == kF32) return moments_s<float>(Q, odd, d, f, mask, F_mom, p, rho, ux, uy, uz, s);
-  if (storage == kF16) return moments_s<_Float16>(Q, odd, d, f, mask, F_mom, p, rho, ux, uy, uz, s);
-  return moments_s<bf16s>(Q, odd, d, f, mask, F_mom, p, rho, ux, uy, uz, s);
+                          const float* F_mom, HydroParams p, uint32_t i0, uint32_t cnt, float* rho, float* ux,
+                          float* uy, float* uz, hipStream_t s) {
+  if (storage == kF32) return moments_s<float>(Q, odd, d, f, mask, F_mom, p, i0, cnt, rho, ux, uy, uz, s);
+  if (storage == kF16) return moments_s<_Float16>(Q, odd, d, f, mask, F_mom, p, i0, cnt, rho, ux, uy, uz, s);
+  return moments_s<bf16s>(Q, odd, d, f, mask, F_mom, p, i0, cnt, rho, ux, uy, uz, s);
 }
 
 template <typename S>

@@ -263,8 +263,8 @@ int scalar_set(const FieldsView& v, ScalarState* s, const float* conc) {
   hipError_t e = hipMalloc((void**)&mom, 4 * N * 4);
   if (e == hipSuccess) e = hipMemcpyAsync(dc, conc, N * 4, hipMemcpyHostToDevice, v.stream);
   if (e == hipSuccess)
-    e = launch_moments(v.Q, v.storage, v.parity, v.d, v.f, v.mask, v.F_mom, v.hp, mom, mom + N, mom + 2 * N,
-                       mom + 3 * N, v.stream);
+    e = launch_moments(v.Q, v.storage, v.parity, v.d, v.f, v.mask, v.F_mom, v.hp, 0, v.d.N, mom, mom + N,
+                       mom + 2 * N, mom + 3 * N, v.stream);
   if (e == hipSuccess) {
     const dim3 g(nblk(N)), b(256);
     if (s->Qs == 7)
@@ -319,8 +319,11 @@ int scalar_put_state(const FieldsView& v, ScalarState* s, const float* h, const 
 int scalar_gather(const FieldsView& v, ScalarState* s, float* conc) {
   int rc = scalar_finish(v, s);
   if (rc) return rc;
-  AUXCHK(v, hipMemcpyAsync(conc, s->C, (size_t)v.d.N * 4, hipMemcpyDeviceToHost, v.stream));
-  AUXCHK(v, hipStreamSynchronize(v.stream));
+  const hipError_t read_back = v.rb->read(v.device, v.stream, 1, [&](int, std::vector<Readback::Seg>& segs) {
+    segs.push_back({conc, s->C, (size_t)v.d.N * 4});
+    return hipSuccess;
+  });
+  AUXCHK(v, read_back);
   return LBM_OK;
 }
 
