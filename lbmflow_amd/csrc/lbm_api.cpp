@@ -122,6 +122,13 @@ struct lbm_fields {
   uint32_t* wale_stats = nullptr;
   bool wale_on = false;
   float wale_cw2 = 0.0f, wale_nut_max = -1.0f;
+  float* wale_work = nullptr;  // cell 0 of the first of its six planes, wale_ps apart
+  size_t wale_ps = 0;
+  // closure inside the step: the omega field's solid cells need their constant
+  bool wale_fill = true;
+  // the last step's scalar step is left to the next step's velocity pass
+  // (inside a span only)
+  bool scalar_pending = false;
   size_t bytes = 0;
 };
 
@@ -446,10 +453,23 @@ int rebuild_mask(lbm_fields* fl) {
   // Fluid on a non-periodic face needs an open-face BC, which is not on this
   // path; stepping such a domain is refused (lbm_run_span).
   fl->open_face_cells = nerr;
+  fl->wale_fill = true;
   fl->probe_built = false;
   int rc2 = count_uncovered(fl);
   if (rc2) return rc2;
   return rebuild_tiles(fl);
+}
+
+// nu of the global rate (les.rs:136-147)
+double wale_nu(const lbm_fields* fl) { return (1.0 / fl->params.omega_p - 0.5) / 3.0; }
+
+// The per-step closure runs inside the collide-stream kernel on closed domains
+// without a uniform force, every neighbour of a fluid cell being inside the
+// domain; periodic and open domains keep the closure's own two passes, which
+// know wrapped and missing neighbours.
+bool wale_in_step(const lbm_fields* fl) {
+  return fl->wale_on && fl->wale_work && !fl->d.per[0] && !fl->d.per[1] && !fl->d.per[2] && !fl->open_face_cells &&
+         !fl->hp.force_on;
 }
 
 // How the tile blocks are dealt to the XCDs (xcd_remap).  A domain whose
@@ -494,6 +514,9 @@ HydroArgs hydro_args(lbm_fields* fl) {
   a.open = fl->open_face_cells ? 1 : 0;
   a.lin = fl->tiles_linear ? 1 : 0;
   a.deal = hydro_deal(fl);
+  if (wale_in_step(fl))
+    a.wale = WaleStep{fl->wale_work, fl->wale_work + 3 * fl->wale_ps, fl->wale_ps, fl->omega, fl->wale_cw2,
+                      (float)wale_nu(fl), fl->wale_nut_max};
   return a;
 }
 
@@ -815,12 +838,14 @@ int lbm_set_params(lbm_fields* fl, const lbm_step_params* p) {
   fl->hp = build_hp(*p);
   fl->collision = p->collision;
   fl->params_set = true;
+  fl->wale_fill = true;
   fl->gen++;
   return LBM_OK;
 }
 
 int lbm_set_omega_field(lbm_fields* fl, const float* omega) {
   if (!fl) return LBM_ERR_INVALID;
+  fl->wale_fill = true;
   const size_t n = fl->d.N;
   if (!omega) {
     HIPCHK(fl->ctx, hipStreamSynchronize(fl->ctx->stream));
@@ -952,8 +977,6 @@ int lbm_read_force_field(lbm_fields* fl, float* ff, int* present) {
 // Laminar viscosity and the f32 quantities WaleLes::update derives from it
 // (les.rs:136-147): nu0, tau0 = 1/2 + 3 nu0, nu_t_max = (tau_eff_max -
 // tau0)/3.
-static double wale_nu(const lbm_fields* fl) { return (1.0 / fl->params.omega_p - 0.5) / 3.0; }
-
 static int wale_coeffs(lbm_fields* fl, double cw, double tau_eff_max, float* cw2, float* nut_max) {
   if (!fl->params_set) return fail(fl->ctx, LBM_ERR_STATE, "set the step parameters before WALE");
   if (!(cw > 0.0) || !std::isfinite(cw)) return fail(fl->ctx, LBM_ERR_INVALID, "WALE coefficient %g", cw);
@@ -982,8 +1005,16 @@ static int wale_buffers(lbm_fields* fl) {
     fl->gen++;
   }
   if (!fl->wale_mom) {
-    int rc = dev_alloc(fl, (void**)&fl->wale_mom, 6 * n * 4);
+    // six planes an odd multiple of 256 elements apart (not all in one HBM
+    // channel), with a guard band of one x-y plane and a row on either side
+    // (WaleStep)
+    const size_t guard = ((size_t)fl->d.nx * fl->d.ny + fl->d.nx + 255) / 256 * 256;
+    size_t ps = (n + 255) / 256 * 256;
+    if (ps / 256 % 2 == 0) ps += 256;
+    int rc = dev_alloc(fl, (void**)&fl->wale_mom, (6 * ps + 2 * guard) * 4);
     if (rc) return rc;
+    fl->wale_ps = ps;
+    fl->wale_work = fl->wale_mom + guard;
   }
   if (!fl->wale_stats) {
     int rc = dev_alloc(fl, (void**)&fl->wale_stats, 2 * sizeof(uint32_t));
@@ -995,12 +1026,17 @@ static int wale_buffers(lbm_fields* fl) {
 // Cached velocity and strain of the current state, then the omega_plus
 // field; launches only (graph-capturable: the statistics words are cleared
 // by a kernel).
+static WaleFields wale_fields(const lbm_fields* fl) {
+  return WaleFields{fl->d,     fl->f,  fl->mask,   fl->wall_u,   fl->field_present ? fl->F_cur : nullptr,
+                    fl->F_mom, fl->hp, fl->parity, fl->open_face_cells ? 1 : 0, (float)(1.0 / fl->params.omega_p), fl->wale_work,
+                    fl->wale_ps};
+}
+
 static int wale_enqueue(lbm_fields* fl, float cw2, float nut_max, float* nut, uint32_t* stats) {
   hipStream_t s = fl->ctx->stream;
-  HIPCHK(fl->ctx, launch_wale(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->wall_u,
-                              fl->field_present ? fl->F_cur : nullptr, fl->F_mom, fl->wale_mom, fl->hp,
-                              (float)(1.0 / fl->params.omega_p),
-                              cw2, (float)wale_nu(fl), nut_max, fl->omega, nut, stats, s));
+  const WaleFields a = wale_fields(fl);
+  HIPCHK(fl->ctx, launch_wale_local(fl->Q, fl->storage, a, nullptr, s));
+  HIPCHK(fl->ctx, launch_wale_omega(a, cw2, (float)wale_nu(fl), nut_max, fl->omega, nut, stats, s));
   return LBM_OK;
 }
 
@@ -1057,6 +1093,7 @@ int lbm_set_wale(lbm_fields* fl, int enabled, double cw, double tau_eff_max) {
   if (!rc) rc = wale_buffers(fl);
   if (rc) return rc;
   fl->wale_on = true;
+  fl->wale_fill = true;
   fl->wale_cw2 = cw2;
   fl->wale_nut_max = nut_max;
   fl->gen++;
@@ -1227,6 +1264,12 @@ static int check_steppable(lbm_fields* fl) {
                 fl->uncovered);
   if (fl->open_face_cells && !fl->scalars.empty())
     return fail(fl->ctx, LBM_ERR_UNSUPPORTED, "scalar distributions do not take open faces on this path");
+  // the closure inside the step writes fluid cells: the others hold the
+  // laminar rate, as the closure's own pass gives it
+  if (fl->wale_fill && wale_in_step(fl)) {
+    HIPCHK(fl->ctx, launch_fill_f32(fl->omega, fl->d.N, 1.0f / (3.0f * (float)wale_nu(fl) + 0.5f), fl->ctx->stream));
+    fl->wale_fill = false;
+  }
   if (!fl->probe_host.empty() && !fl->probe_built) return probe_build(fl);
   return LBM_OK;
 }
@@ -1385,11 +1428,30 @@ static int open_faces_step(lbm_fields* fl) {
   return LBM_OK;
 }
 
+// Whether a step may leave its scalar step to the next step's velocity pass:
+// a single D3Q7 scalar beside the closure inside the step.
+static bool scalar_rides(const lbm_fields* fl) {
+  int Qs = 0;
+  double D = 0.0;
+  if (fl->scalars.size() != 1 || !wale_in_step(fl)) return false;
+  scalar_info(fl->scalars[0], &Qs, &D);
+  return Qs == 7;
+}
+
 // One collide-stream step (main kernel, forced-cell list kernel) plus the
-// scalar distributions; launches only.
+// scalar distributions; launches only.  A scalar step that rides on the next
+// step's velocity pass is run by finish_scalars at the end of the span.
 static int hydro_step(lbm_fields* fl) {
   hipStream_t s = fl->ctx->stream;
-  if (fl->wale_on) {
+  if (wale_in_step(fl)) {
+    ScalarStepArgs sc;
+    if (fl->scalar_pending) {
+      int rc = scalar_turn(view_of(fl), fl->scalars[0], &sc);
+      if (rc) return rc;
+    }
+    HIPCHK(fl->ctx, launch_wale_local(fl->Q, fl->storage, wale_fields(fl), fl->scalar_pending ? &sc : nullptr, s));
+    fl->scalar_pending = false;
+  } else if (fl->wale_on) {
     int rc = wale_enqueue(fl, fl->wale_cw2, fl->wale_nut_max, nullptr, nullptr);
     if (rc) return rc;
   }
@@ -1432,6 +1494,10 @@ static int hydro_step(lbm_fields* fl) {
   }
   fl->parity ^= 1;
   fl->time += 1;
+  if (scalar_rides(fl)) {
+    fl->scalar_pending = true;
+    return LBM_OK;
+  }
   for (ScalarState* sc : fl->scalars) {
     int rc = scalar_step(view_of(fl), sc);
     if (rc) return rc;
@@ -1439,8 +1505,14 @@ static int hydro_step(lbm_fields* fl) {
   return LBM_OK;
 }
 
-// The concentrations of the state a span ends with.
+// What a span ends with: the last step's scalar step, if it was left to a
+// step that does not come, and the concentrations.
 static int finish_scalars(lbm_fields* fl) {
+  if (fl->scalar_pending) {
+    fl->scalar_pending = false;
+    int rc = scalar_step(view_of(fl), fl->scalars[0]);
+    if (rc) return rc;
+  }
   for (ScalarState* sc : fl->scalars) {
     int rc = scalar_finish(view_of(fl), sc);
     if (rc) return rc;
@@ -1512,7 +1584,7 @@ int lbm_run_ibm_span(lbm_fields* fl, int steps, int use_graph, double* torque, l
       if (!scalar_steady(sc)) return false;
     return true;
   };
-  for (; use_graph && k < steps && !steady(); ++k) {
+  for (; use_graph && k < steps && (!steady() || scalar_rides(fl) != fl->scalar_pending); ++k) {
     rc = ibm_step(fl);
     if (rc) return rc;
   }
@@ -2302,6 +2374,7 @@ int lbm_autotune_tiles(lbm_fields* fl, int trial_steps, uint32_t zb_out[2], doub
     if (rc) break;
     HydroArgs a = hydro_args(fl);
     a.f = (char*)copy + off;
+    a.wale = WaleStep{};  // a trial writes no omega field
     const int p0 = fl->parity;
     double sum[2] = {0.0, 0.0};
     // one untimed pair, then T launches with an event between each

@@ -100,6 +100,9 @@ void scalar_destroy(ScalarState* s);
 int scalar_set(const FieldsView& v, ScalarState* s, const float* conc);
 int scalar_gather(const FieldsView& v, ScalarState* s, float* conc);
 int scalar_step(const FieldsView& v, ScalarState* s);
+// This step's buffers for a kernel that runs it elsewhere; the state moves on
+// as scalar_step moves it.
+int scalar_turn(const FieldsView& v, ScalarState* s, ScalarStepArgs* st);
 int scalar_finish(const FieldsView& v, ScalarState* s);
 int scalar_settle(const FieldsView& v, ScalarState* s);
 // whether a step launches the same kernels as the next one (false right

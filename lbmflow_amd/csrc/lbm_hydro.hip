@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "lbm_device.hpp"
+#include "lbm_wale.hpp"
 
 namespace lbm {
 
@@ -649,7 +650,10 @@ __device__ __forceinline__ void slot_st(S* p, float v) {
 //
 // PLAIN: the whole tile is fluid with mask word 0 (no wall link, no force
 // list, no moving wall), known from the tile list; the mask is not read.
-template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool FILL, bool PLAIN = false>
+// WALE: the relaxation rate comes from the closure (lbm_wale.hpp), taken here
+// from the neighbours' cached velocities and written to the omega field.
+template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool FILL, bool PLAIN = false,
+          bool WALE = false>
 __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32_t x, uint32_t y, uint32_t z,
                                           const uint32_t* mask_ptr, uint32_t skip, const float Fm[3],
                                           const float Fc[3], uint32_t xlo = 0u, uint32_t xhi = 0u,
@@ -662,14 +666,31 @@ __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32
   // predicated on it.
   const uint32_t m = PLAIN ? 0u : *mask_ptr;
   float fv[Q];
-  sfor<0, Q>([&](auto qc) {
+  [[maybe_unused]] float wale_om = 0.0f;
+  auto slot = [&](auto qc) {
     constexpr int q = decltype(qc)::value;
     constexpr int o = lat_opp(q);
     if constexpr (!ODD)
-      fv[q] = slot_ld<S, Q, q>(sl.template at<q, 0, 0, 0>());
+      return (const S*)sl.template at<q, 0, 0, 0>();
     else
-      fv[q] = slot_ld<S, Q, q>(sl.template at<o, -lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>());
-  });
+      return (const S*)sl.template at<o, -lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>();
+  };
+  if constexpr (WALE) {
+    // The closure's loads go first and the rate is computed while the
+    // populations are still on their way, so it costs the step neither a
+    // latency nor a register of its peak.  The fence keeps every load ahead of
+    // the first use: without it the scheduler meets the register limit by
+    // waiting for each 16-bit load before the next (512^3 fp16 odd step 5.11
+    // ms against 3.24).
+    WaleLoads<PLAIN> wl(a.wale, a.d, i);
+    S raw[Q];
+    sfor<0, Q>([&](auto qc) { raw[decltype(qc)::value] = *slot(qc); });
+    __builtin_amdgcn_sched_barrier(0);
+    if (!(m & kMaskSolid)) wale_om = wl.omega(a.wale, a.d, a.wall_u, i, m);
+    sfor<0, Q>([&](auto qc) { fv[decltype(qc)::value] = slot_ld<S, Q, decltype(qc)::value>(&raw[decltype(qc)::value]); });
+  } else {
+    sfor<0, Q>([&](auto qc) { fv[decltype(qc)::value] = slot_ld<S, Q, decltype(qc)::value>(slot(qc)); });
+  }
   // Consume every loaded value before the solid test, so the compiler cannot
   // sink the population loads behind the mask branch: one memory latency per
   // cell instead of two.
@@ -710,10 +731,12 @@ __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32
     }
   }
   float op = a.p.omega_p, cp = a.p.cp, os = a.p.omega_shear;
-  if (a.omega) {  // per-cell omega_plus (kernels.rs:151-156)
-    op = a.omega[i];
+  if (WALE || a.omega) {  // per-cell omega_plus (kernels.rs:151-156)
+    op = WALE ? wale_om : a.omega[i];
     cp = 1.0f - op / 2.0f;
     os = op;
+    if constexpr (WALE)
+      if (!dead) a.wale.omega[i] = op;
   }
   float r;
   if constexpr (KIND == 0) {
@@ -800,8 +823,8 @@ __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32
   }
 }
 
-template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP>
-__global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
+template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool WALE>
+__device__ __forceinline__ void hydro_tile(const HydroArgs& a) {
   // each wave takes one active 64-cell tile; tiles of only solid (or
   // force-listed) cells are never launched
   const uint32_t b = xcd_remap(blockIdx.x, gridDim.x, a.deal);
@@ -815,12 +838,12 @@ __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
     const uint32_t i = tile * 64 + (threadIdx.x & 63);
     if (i >= a.d.N || (te & ((threadIdx.x & 32) ? kTileDeadHi : kTileDeadLo))) return;
     if (te & kTilePlain) {
-      cell_step<Q, S, KIND, ODD, FON, WRAP, true, true>(a, i, 0u, 0u, 0u, nullptr, 0u, a.p.F, a.p.F);
+      cell_step<Q, S, KIND, ODD, FON, WRAP, true, true, WALE>(a, i, 0u, 0u, 0u, nullptr, 0u, a.p.F, a.p.F);
     } else {
       const uint32_t c0 = tile * 64;
       const uint32_t lo = (te & kTileDeadLo) ? c0 + 32 : c0;
       const uint32_t hi = min((te & kTileDeadHi) ? c0 + 31 : c0 + 63, a.d.N - 1);
-      cell_step<Q, S, KIND, ODD, FON, WRAP, true, false>(a, i, 0u, 0u, 0u, a.mask + i, kMaskSolid | kMaskForced,
+      cell_step<Q, S, KIND, ODD, FON, WRAP, true, false, WALE>(a, i, 0u, 0u, 0u, a.mask + i, kMaskSolid | kMaskForced,
                                                          a.p.F, a.p.F, lo, hi, i);
     }
     return;
@@ -831,15 +854,36 @@ __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
   const uint32_t y = row % a.d.ny, z = row / a.d.ny;
   const uint32_t i = row * a.d.nx + x;
   if (te & kTilePlain) {
-    cell_step<Q, S, KIND, ODD, FON, WRAP, true, true>(a, i, x, y, z, nullptr, 0u, a.p.F, a.p.F);
+    cell_step<Q, S, KIND, ODD, FON, WRAP, true, true, WALE>(a, i, x, y, z, nullptr, 0u, a.p.F, a.p.F);
   } else {
     // the tile's live x range (an all-solid half is not visited)
     const uint32_t x0 = seg * 64;
     const uint32_t xlo = (te & kTileDeadLo) ? x0 + 32 : x0;
     const uint32_t xhi = min((te & kTileDeadHi) ? x0 + 31 : x0 + 63, a.d.nx - 1);
-    cell_step<Q, S, KIND, ODD, FON, WRAP, true, false>(a, i, x, y, z, a.mask + i, kMaskSolid | kMaskForced,
+    cell_step<Q, S, KIND, ODD, FON, WRAP, true, false, WALE>(a, i, x, y, z, a.mask + i, kMaskSolid | kMaskForced,
                                                        a.p.F, a.p.F, xlo, xhi);
   }
+}
+
+template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP>
+__global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
+  hydro_tile<Q, S, KIND, ODD, FON, WRAP, false>(a);
+}
+
+// The step with the WALE closure inside (closed domains, no uniform force):
+// the gradient, nu_t and omega_plus of each cell it updates, instead of a pass
+// of their own that writes an omega field for this kernel to read.  The
+// velocities of the neighbours come from L2 (18 loads); what is added from HBM
+// is what that pass read (24 bytes per cell), what is saved is its launch, its
+// masks and its waiting: it was bound by VALU and latency, and here both hide
+// under the populations' loads.  Four waves per SIMD as k_hydro has.
+// Per step, closure and collide-stream: 256^3 D3Q27 fp32 1.153 -> 1.094 ms (the
+// velocity pass 0.365, this kernel 0.705 / 0.753); 512^3 fp16 with a D3Q7
+// tracer taken along by that pass 8.31 -> 6.62 ms (3.20, and 3.13 / 3.70 here,
+// where nu_t's 380 VALU instructions per wave make it VALU-bound).
+template <int Q, typename S, int KIND, bool ODD>
+__global__ __launch_bounds__(256, 4) void k_hydro_wale(HydroArgs a) {
+  hydro_tile<Q, S, KIND, ODD, false, false, true>(a);
 }
 
 // Cells carrying a per-cell force: the velocity uses the force of the cached
@@ -847,7 +891,7 @@ __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
 // current field (F_cur), as the reference's stale-moment step does
 // (solver.rs:2805-2822 keeps moments across a non-uniform clear).  After the
 // step the cached moments carry F_cur.
-template <int Q, typename S, int KIND, bool ODD>
+template <int Q, typename S, int KIND, bool ODD, bool WALE = false>
 __device__ __forceinline__ void list_cell(const HydroArgs& a, uint32_t i) {
   const uint32_t m = a.mask[i];
   if (m & kMaskSolid) return;
@@ -859,16 +903,16 @@ __device__ __forceinline__ void list_cell(const HydroArgs& a, uint32_t i) {
     Fm[c] = a.p.F[c] + a.F_mom[3 * (size_t)i + c];
     Fc[c] = a.p.F[c] + a.F_cur[3 * (size_t)i + c];
   }
-  cell_step<Q, S, KIND, ODD, true, true, false>(a, i, x, y, z, a.mask + i, kMaskSolid, Fm, Fc);
+  cell_step<Q, S, KIND, ODD, true, true, false, false, WALE>(a, i, x, y, z, a.mask + i, kMaskSolid, Fm, Fc);
 #pragma unroll
   for (int c = 0; c < 3; ++c) a.F_mom[3 * (size_t)i + c] = a.F_cur[3 * (size_t)i + c];
 }
 
-template <int Q, typename S, int KIND, bool ODD>
+template <int Q, typename S, int KIND, bool ODD, bool WALE = false>
 __global__ __launch_bounds__(256) void k_hydro_list(HydroArgs a) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.nlist) return;
-  list_cell<Q, S, KIND, ODD>(a, a.flist[k]);
+  list_cell<Q, S, KIND, ODD, WALE>(a, a.flist[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -938,7 +982,12 @@ static hipError_t hydro_q(int odd, const HydroArgs& a, hipStream_t s, bool list)
   if (list) {
     if (a.nlist == 0) return hipSuccess;
     const dim3 grid(blocks_for(a.nlist)), block(256);
-    if (odd)
+    if (a.wale.vel) {
+      if (odd)
+        hipLaunchKernelGGL((k_hydro_list<Q, S, KIND, true, true>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_hydro_list<Q, S, KIND, false, true>), grid, block, 0, s, a);
+    } else if (odd)
       hipLaunchKernelGGL((k_hydro_list<Q, S, KIND, true>), grid, block, 0, s, a);
     else
       hipLaunchKernelGGL((k_hydro_list<Q, S, KIND, false>), grid, block, 0, s, a);
@@ -948,6 +997,14 @@ static hipError_t hydro_q(int odd, const HydroArgs& a, hipStream_t s, bool list)
   const dim3 grid((a.ntiles + 3) / 4), block(256);
   const bool fon = a.p.force_on != 0;
   const bool wrap = a.d.per[0] || a.d.per[1] || a.d.per[2] || a.open;
+  if (a.wale.vel) {  // closed domains without a uniform force (wale_in_step)
+    if (fon || wrap) return hipErrorInvalidValue;
+    if (odd)
+      hipLaunchKernelGGL((k_hydro_wale<Q, S, KIND, true>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((k_hydro_wale<Q, S, KIND, false>), grid, block, 0, s, a);
+    return hipGetLastError();
+  }
   const int sel = (odd ? 4 : 0) | (fon ? 2 : 0) | (wrap ? 1 : 0);
   switch (sel) {
     case 0: hipLaunchKernelGGL((k_hydro<Q, S, KIND, false, false, false>), grid, block, 0, s, a); break;

@@ -49,6 +49,22 @@ struct HydroParams {
   int force_on;      // F != 0
 };
 
+// Per-step WALE closure inside the collide-stream kernels (lbm_wale.hpp): the
+// cached velocity and strain of the state before the step (k_wale_local) and
+// the closure's coefficients.  `vel` and `strain` point at cell 0 of three
+// planes `ps` apart each, the six in one allocation with a guard band of one
+// x-y plane and a row on both sides, so that the neighbours of a solid face
+// cell stay inside it.
+struct WaleStep {
+  const float* vel;  // null: no per-step closure
+  const float* strain;
+  size_t ps;
+  float* omega;       // omega_plus out
+  float cw_delta_sq;  // (Cw Delta)^2
+  float nu0, nut_max; // laminar viscosity; < 0: no clip
+  float pad = 0.0f;
+};
+
 struct HydroArgs {
   Dom d;
   Tiling t;
@@ -67,6 +83,7 @@ struct HydroArgs {
   uint32_t nlist;
   float* F_mom;             // N x 3: force of the cached moments
   const float* F_cur;       // N x 3: current field
+  WaleStep wale;            // per-step closure inside the step (vel null: none)
   int open;                 // fluid on a non-periodic (open) face: wrap every offset
   uint32_t deal;            // how the tile blocks are dealt to the XCDs (xcd_remap)
   int lin;                  // tiles are 64-cell blocks of the linear index (no axis wraps)
@@ -204,14 +221,38 @@ hipError_t launch_probe(int Q, int storage, int post, const ProbeArgs& a, hipStr
 hipError_t launch_open_faces(int Q, int storage, const FaceArgs& a, hipStream_t s);
 hipError_t launch_uncovered(const Dom& d, const uint8_t* solid, uint32_t open_bits, unsigned int* count,
                             hipStream_t s);
-// WALE omega_plus field from the state and its cached moments `mom` (4 x N:
-// rho, ux, uy, uz) (lbm_les.hip).  `stats` (2 words, cleared here by a
-// kernel): clipped cell count, bits of the largest raw nu_t.
-// work: 6 x N floats (cached velocity, off-diagonal strain)
-hipError_t launch_wale(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
-                       const float* wall_u, const float* F_cur, const float* F_mom, float* work, const HydroParams& p,
-                       float tau_eff, float cw_delta_sq, float nu0, float nut_max, float* omega, float* nut,
-                       uint32_t* stats, hipStream_t s);
+// WALE (lbm_les.hip): cached velocity and off-diagonal strain of the state
+// into six planes `ps` apart at `work`, and the omega_plus field from them.
+// `stats` (2 words, cleared here by a kernel): clipped cell count, bits of the
+// largest raw nu_t.
+struct WaleFields {
+  Dom d;
+  const void* f;
+  const uint32_t* mask;
+  const float* wall_u;  // N x 3 or null (velocity of each solid cell's wall)
+  const float* F_cur;   // N x 3 or null (current force field, nonzero only on
+                        // the force list, whose fluid cells carry kMaskForced)
+  const float* F_mom;   // N x 3 or null (the field the cached moments were taken with)
+  HydroParams p;        // the uniform force
+  int odd;
+  int open;       // fluid on a non-periodic (open) face: offsets wrap
+  float tau_eff;  // 1/omega_p of the global rate (stress scale)
+  float* work;    // ux, uy, uz, Sxy, Sxz, Syz
+  size_t ps;
+};
+struct ScalarStepArgs;
+// sc: the previous step's D3Q7 scalar step, taken along (closed domains)
+hipError_t launch_wale_local(int Q, int storage, const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s);
+hipError_t launch_wale_omega(const WaleFields& a, float cw_delta_sq, float nu0, float nut_max, float* omega,
+                             float* nut, uint32_t* stats, hipStream_t s);
+// One passive-scalar step of a domain (lbm_scalar.hpp).
+struct ScalarStepArgs {
+  const float* h;   // Qs planes: this step's distribution
+  float* h2;        // Qs planes: the next one
+  const float* C;   // concentration to collide with, null: the sum of h
+  size_t ps;        // plane stride
+  float omega;
+};
 hipError_t launch_build_mask(int Q, const Dom& d, const uint8_t* solid, const float* wall_u, uint32_t* mask,
                              unsigned int* err_count, hipStream_t s);
 hipError_t launch_mark_forced(const uint32_t* flist, uint32_t n, uint32_t* mask, hipStream_t s);

@@ -15,94 +15,71 @@
 //     The second pass marches (x, y) columns along z with the z - 1, z,
 //     z + 1 velocities in registers, so each velocity is read from memory
 //     once; x and y neighbours come from the tile's own rows in L2.
+// On closed domains the per-step closure does without the second pass: the
+// collide-stream kernel takes the same gradient and nu_t of each cell it
+// updates (lbm_wale.hpp).
 // Bytes per fluid cell: 4Q + 4 (mask) + 24 in the first pass; 4 + 24 + the
 // neighbours' velocities (mostly from L2) + 4 in the second, against two
 // full population reads for a moment pass followed by a strain pass.
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
+#include "lbm_scalar.hpp"
+#include "lbm_wale.hpp"
 
 #pragma clang fp contract(off)
 
 namespace lbm {
 
-struct WaleArgs {
-  Dom d;
-  const void* f;
-  const uint32_t* mask;
-  const float* wall_u;  // N x 3 or null (velocity of each solid cell's wall)
-  const float* F_cur;   // N x 3 or null (current force field, nonzero only on
-                        // the force list, whose fluid cells carry kMaskForced)
-  const float* F_mom;   // N x 3 or null (the field the cached moments were taken with)
-  HydroParams p;        // the uniform force
-  int odd;
-  float tau_eff;      // 1/omega_p of the global rate (stress scale)
+// what the second pass computes with and writes
+struct WaleOut {
   float cw_delta_sq;  // (Cw Delta)^2
   float nu0;          // laminar viscosity
   float nut_max;      // < 0: no clip
-  float* vel;         // 3 x N: ux, uy, uz of the current state (cached moments)
-  float* strain;      // 3 x N: Sxy, Sxz, Syz from the non-equilibrium stress
-  float* omega;       // N: omega_plus out
-  float* nut;         // N or null: nu_t out (after the clip)
+  float* omega;       // N: omega_plus
+  float* nut;         // N or null: nu_t (after the clip)
   uint32_t* stats;    // null or [clipped cells, bits of the largest raw nu_t]
-  uint32_t zlen;      // cells each thread of the second pass marches along z
 };
 
-// Population loads marked non-temporal: each population is read once, so
-// the L2 is left to the velocity planes the neighbour differences reuse.
-template <typename S>
-__device__ __forceinline__ float ld_nt(const S* p, uint32_t i);
-template <>
-__device__ __forceinline__ float ld_nt<float>(const float* p, uint32_t i) {
-  return __builtin_nontemporal_load(p + i);
-}
-template <>
-__device__ __forceinline__ float ld_nt<_Float16>(const _Float16* p, uint32_t i) {
-  return (float)__builtin_nontemporal_load(p + i);
-}
-template <>
-__device__ __forceinline__ float ld_nt<bf16s>(const bf16s* p, uint32_t i) {
-  const uint16_t v = __builtin_nontemporal_load((const uint16_t*)p + i);
-  return __uint_as_float((uint32_t)v << 16);
-}
+// fp32 populations of the first pass are loaded non-temporally: each is read
+// once, and the L2 is left to the velocity planes (256^3 D3Q27 0.417 -> 0.365
+// ms; the step after it reads its populations from memory again either way).
+// 16-bit ones are faster through L2, whose lines two neighbouring odd-state
+// tiles share (512^3 fp16 2.07 -> 1.86 ms, with a scalar 3.48 -> 3.20).
 template <int Q, typename S, int q>
-__device__ __forceinline__ float read_pop_nt(const S* base, size_t ps, const Nbr& nb, uint32_t i, uint32_t m,
-                                             bool odd) {
-  constexpr int o = lat_opp(q);
-  const S* plane;
-  uint32_t j;
-  if (!odd || ((m >> q) & 1u)) {
-    plane = base + (size_t)q * ps;
-    j = i;
+__device__ __forceinline__ float read_pop_once(const S* base, size_t ps, const Nbr& nb, uint32_t i, uint32_t m,
+                                               bool odd) {
+  if constexpr (sizeof(S) == 4) {
+    const bool own = !odd || ((m >> q) & 1u);
+    const uint32_t j = own ? i : i + (uint32_t)nb.template off<-lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>();
+    return __builtin_nontemporal_load(base + (size_t)(own ? q : lat_opp(q)) * ps + j);
   } else {
-    plane = base + (size_t)o * ps;
-    j = i + (uint32_t)nb.template off<-lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>();
+    return read_pop<Q, S, q>(base, ps, nb, i, m, odd);
   }
-  float v = ld_nt<S>(plane, j);
-  if constexpr (Store<S>::kScaled) v = v * lat_wf(Q, q);
-  return v;
 }
 
 // Pass 1, per cell: the cached moments (moments_row with the force the state
 // was produced under, as the moment readback computes them) and the
 // off-diagonal strain from the same populations, read once.
-template <int Q, typename S>
-__global__ __launch_bounds__(256) void k_wale_local(WaleArgs a) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// A solid cell's values are never read (a solid neighbour contributes its
+// wall velocity).  With QS the pass takes the previous step's passive-scalar
+// step along (no axis wraps then): it collides with exactly these velocities,
+// so its own read of the populations (Q S bytes per cell) is saved.
+template <int Q, typename S, bool WRAP, int QS>
+__global__ __launch_bounds__(256) void k_wale_local(WaleFields a, uint32_t deal, ScalarStepArgs sc) {
+  const uint32_t i = xcd_remap(blockIdx.x, gridDim.x, deal) * 256 + threadIdx.x;
   if (i >= a.d.N) return;
-  const size_t N = a.d.N;
+  float* const vel = a.work;
+  float* const strain = a.work + 3 * a.ps;
   const uint32_t m = a.mask[i];
-  if (m & kMaskSolid) {
-    a.vel[i] = a.vel[N + i] = a.vel[2 * N + i] = 0.0f;
-    a.strain[i] = a.strain[N + i] = a.strain[2 * N + i] = 0.0f;
-    return;
-  }
-  uint32_t x, y, z;
-  cell_xyz(a.d, i, x, y, z);
-  const Nbr nb(a.d, x, y, z);
-  float fv[Q];
+  if (m & kMaskSolid) return;
+  uint32_t x = 0, y = 0, z = 0;
+  if constexpr (WRAP) cell_xyz(a.d, i, x, y, z);
+  const Nbr nb = WRAP ? Nbr(a.d, x, y, z) : Nbr(a.d);
+  float hv[QS > 0 ? QS : 1], fv[Q];
+  if constexpr (QS > 0) scalar_load<QS>(sc, i, hv);
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    fv[q] = read_pop_nt<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, a.odd != 0);
+    fv[q] = read_pop_once<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, a.odd != 0);
   });
   float Fm[3] = {a.p.F[0], a.p.F[1], a.p.F[2]};
   bool fon = a.p.force_on != 0;
@@ -112,9 +89,10 @@ __global__ __launch_bounds__(256) void k_wale_local(WaleArgs a) {
   }
   float r, u0, u1, u2;
   moments<Q>(fv, Fm, fon, r, u0, u1, u2);
-  a.vel[i] = u0;
-  a.vel[N + i] = u1;
-  a.vel[2 * N + i] = u2;
+  vel[i] = u0;
+  vel[a.ps + i] = u1;
+  vel[2 * a.ps + i] = u2;
+  if constexpr (QS > 0) scalar_push<QS>(sc, nb, i, m, hv, u0, u1, u2);
   // Pi_neq = sum_q c c (f_q - feq_q), deviation-form equilibrium
   // (kernels.rs:103-121); terms with a zero factor add exact zeros in the
   // reference's sums and are dropped.
@@ -147,14 +125,14 @@ __global__ __launch_bounds__(256) void k_wale_local(WaleArgs a) {
   pyz = pyz + 0.5f * (u1 * F2 + u2 * F1);
   // S = -Pi / (2 cs^2 rho tau), tau = 1/omega_p (the global rate)
   const float scale = -(1.0f / ((2.0f / 3.0f) * r * a.tau_eff));
-  a.strain[i] = pxy * scale;
-  a.strain[N + i] = pxz * scale;
-  a.strain[2 * N + i] = pyz * scale;
+  strain[i] = pxy * scale;
+  strain[a.ps + i] = pxz * scale;
+  strain[2 * a.ps + i] = pyz * scale;
 }
 
 // One neighbour of a finite difference: kind 0 none (non-periodic domain
 // face), 1 fluid (v = its cached velocity), 2 solid (v = its wall velocity).
-__device__ __forceinline__ int wale_nbr(const WaleArgs& a, bool none, uint32_t j, uint32_t mj, const float* uj,
+__device__ __forceinline__ int wale_nbr(const WaleFields& a, bool none, uint32_t j, uint32_t mj, const float* uj,
                                         float v[3]) {
   if (none) {
     v[0] = v[1] = v[2] = 0.0f;
@@ -176,78 +154,6 @@ __device__ __forceinline__ int wale_nbr(const WaleArgs& a, bool none, uint32_t j
   return 1;
 }
 
-// nu_t of one fluid cell from its velocity, strain and the neighbours of
-// each axis (kp/km kinds, pv/mv values)
-__device__ __forceinline__ float wale_nut(const WaleArgs& a, const float own[3], float sxy, float sxz, float syz,
-                                          const int kp[3], const int km[3], const float pv[3][3],
-                                          const float mv[3][3]) {
-  float fd[3][3];
-  const bool central = kp[0] == 1 && km[0] == 1 && kp[1] == 1 && km[1] == 1 && kp[2] == 1 && km[2] == 1;
-  if (central) {  // every neighbour fluid: the common case
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) fd[k][ax] = (pv[ax][k] - mv[ax][k]) * 0.5f;
-  } else {
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax)
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float v = 0.0f;
-      if (kp[ax] == 1 && km[ax] == 1)
-        v = (pv[ax][k] - mv[ax][k]) * 0.5f;
-      else if (kp[ax] == 1 && km[ax] == 2)
-        v = -(4.0f / 3.0f) * mv[ax][k] + own[k] + (1.0f / 3.0f) * pv[ax][k];
-      else if (kp[ax] == 2 && km[ax] == 1)
-        v = (4.0f / 3.0f) * pv[ax][k] - own[k] - (1.0f / 3.0f) * mv[ax][k];
-      else if (kp[ax] == 1 && km[ax] == 0)
-        v = pv[ax][k] - own[k];
-      else if (kp[ax] == 0 && km[ax] == 1)
-        v = own[k] - mv[ax][k];
-      fd[k][ax] = v;
-    }
-  }
-  float g[3][3];
-  g[0][0] = fd[0][0];
-  g[1][1] = fd[1][1];
-  g[2][2] = fd[2][2];
-  g[0][1] = sxy + 0.5f * (fd[0][1] - fd[1][0]);
-  g[1][0] = sxy + 0.5f * (fd[1][0] - fd[0][1]);
-  g[0][2] = sxz + 0.5f * (fd[0][2] - fd[2][0]);
-  g[2][0] = sxz + 0.5f * (fd[2][0] - fd[0][2]);
-  g[1][2] = syz + 0.5f * (fd[1][2] - fd[2][1]);
-  g[2][1] = syz + 0.5f * (fd[2][1] - fd[1][2]);
-  // WALE invariants
-  float s2 = 0.0f, g2[3][3];
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const float sv = 0.5f * (g[p][q] + g[q][p]);
-      s2 = s2 + sv * sv;
-      float acc = 0.0f;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) acc = acc + g[p][k] * g[k][q];
-      g2[p][q] = acc;
-    }
-  const float tr = g2[0][0] + g2[1][1] + g2[2][2];
-  float sd2 = 0.0f;
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      float sd = 0.5f * (g2[p][q] + g2[q][p]);
-      if (p == q) sd = sd - tr / 3.0f;
-      sd2 = sd2 + sd * sd;
-    }
-  // the three powers from square roots (s2^2.5 = s2^2 sqrt(s2),
-  // sd2^1.5 = sd2 sqrt(sd2), sd2^1.25 = sd2 sqrt(sqrt(sd2))): a few ulp from
-  // the correctly rounded powers, at a fraction of a general powf's cost
-  const float rs = sqrtf(s2), rd = sqrtf(sd2);
-  const float denom = s2 * s2 * rs + sd2 * sqrtf(rd);
-  return denom > 0.0f ? a.cw_delta_sq * (sd2 * rd) / denom : 0.0f;
-}
-
 // Pass 2: a block is a 64 x 4 tile of (x, y) columns, each thread marches
 // its column over `zlen` cells keeping the mask and cached velocity of
 // z - 1, z, z + 1 in registers, so every velocity is read from HBM about
@@ -257,14 +163,15 @@ __device__ __forceinline__ float wale_nut(const WaleArgs& a, const float own[3],
 constexpr uint32_t kWaleTileX = 64, kWaleTileY = 4;
 static_assert(kWaleTileX * kWaleTileY == 256 && kWaleTileX == 64, "one wave per tile row, 256-thread blocks");
 
-template <int Q, typename S>
-__global__ __launch_bounds__(256) void k_wale(WaleArgs a) {
+__global__ __launch_bounds__(256) void k_wale(WaleFields a, WaleOut o, uint32_t zlen) {
+  const float* const vel = a.work;
+  const float* const strain = a.work + 3 * a.ps;
   const uint32_t nx = a.d.nx, ny = a.d.ny, nz = a.d.nz;
   const uint32_t x = blockIdx.x * kWaleTileX + (threadIdx.x & (kWaleTileX - 1));
   const uint32_t y = blockIdx.y * kWaleTileY + threadIdx.x / kWaleTileX;
-  const uint32_t z0 = blockIdx.z * a.zlen;
-  const uint32_t z1 = min(z0 + a.zlen, nz);
-  const size_t N = a.d.N;
+  const uint32_t z0 = blockIdx.z * zlen;
+  const uint32_t z1 = min(z0 + zlen, nz);
+  const size_t N = a.ps;
   const uint32_t plane = nx * ny;
   uint32_t cnt = 0u, mx = 0u;
   if (x < nx && y < ny && z0 < nz) {
@@ -272,12 +179,12 @@ __global__ __launch_bounds__(256) void k_wale(WaleArgs a) {
     const uint32_t iwrap = (nz - 1) * plane;  // z = 0 <-> z = nz - 1
     uint32_t jm = z0 == 0 ? i + iwrap : i - plane;
     uint32_t mm = a.mask[jm], mc = a.mask[i];
-    float um[3] = {a.vel[jm], a.vel[N + jm], a.vel[2 * N + jm]};
-    float uc[3] = {a.vel[i], a.vel[N + i], a.vel[2 * N + i]};
+    float um[3] = {vel[jm], vel[N + jm], vel[2 * N + jm]};
+    float uc[3] = {vel[i], vel[N + i], vel[2 * N + i]};
     for (uint32_t z = z0; z < z1; ++z) {
       const uint32_t jp = z == nz - 1 ? i - iwrap : i + plane;
       const uint32_t mp = a.mask[jp];
-      const float up[3] = {a.vel[jp], a.vel[N + jp], a.vel[2 * N + jp]};
+      const float up[3] = {vel[jp], vel[N + jp], vel[2 * N + jp]};
       float nut_raw = 0.0f;
       if (!(mc & kMaskSolid)) {
         const Nbr nb(a.d, x, y, z);
@@ -285,26 +192,26 @@ __global__ __launch_bounds__(256) void k_wale(WaleArgs a) {
         float pv[3][3], mv[3][3];
         {
           const uint32_t j1 = i + (uint32_t)nb.xp, j2 = i + (uint32_t)nb.xm;
-          const float u1[3] = {a.vel[j1], a.vel[N + j1], a.vel[2 * N + j1]};
-          const float u2[3] = {a.vel[j2], a.vel[N + j2], a.vel[2 * N + j2]};
+          const float u1[3] = {vel[j1], vel[N + j1], vel[2 * N + j1]};
+          const float u2[3] = {vel[j2], vel[N + j2], vel[2 * N + j2]};
           kp[0] = wale_nbr(a, x == nx - 1 && !a.d.per[0], j1, a.mask[j1], u1, pv[0]);
           km[0] = wale_nbr(a, x == 0 && !a.d.per[0], j2, a.mask[j2], u2, mv[0]);
         }
         {
           const uint32_t j1 = i + (uint32_t)nb.yp, j2 = i + (uint32_t)nb.ym;
-          const float u1[3] = {a.vel[j1], a.vel[N + j1], a.vel[2 * N + j1]};
-          const float u2[3] = {a.vel[j2], a.vel[N + j2], a.vel[2 * N + j2]};
+          const float u1[3] = {vel[j1], vel[N + j1], vel[2 * N + j1]};
+          const float u2[3] = {vel[j2], vel[N + j2], vel[2 * N + j2]};
           kp[1] = wale_nbr(a, y == ny - 1 && !a.d.per[1], j1, a.mask[j1], u1, pv[1]);
           km[1] = wale_nbr(a, y == 0 && !a.d.per[1], j2, a.mask[j2], u2, mv[1]);
         }
         kp[2] = wale_nbr(a, z == nz - 1 && !a.d.per[2], jp, mp, up, pv[2]);
         km[2] = wale_nbr(a, z == 0 && !a.d.per[2], jm, mm, um, mv[2]);
-        nut_raw = wale_nut(a, uc, a.strain[i], a.strain[N + i], a.strain[2 * N + i], kp, km, pv, mv);
+        nut_raw = wale_nut<false>(o.cw_delta_sq, uc, strain[i], strain[N + i], strain[2 * N + i], kp, km, pv, mv);
       }
-      const bool clipped = a.nut_max >= 0.0f && nut_raw > a.nut_max;
-      const float nut = clipped ? a.nut_max : nut_raw;
-      a.omega[i] = 1.0f / (3.0f * (a.nu0 + nut) + 0.5f);
-      if (a.nut) a.nut[i] = nut;
+      const bool clipped = o.nut_max >= 0.0f && nut_raw > o.nut_max;
+      const float nut = clipped ? o.nut_max : nut_raw;
+      o.omega[i] = wale_omega(o.nu0, nut);
+      if (o.nut) o.nut[i] = nut;
       cnt += clipped ? 1u : 0u;
       mx = max(mx, __float_as_uint(nut_raw));
       // slide the window one cell up
@@ -320,14 +227,14 @@ __global__ __launch_bounds__(256) void k_wale(WaleArgs a) {
       uc[2] = up[2];
     }
   }
-  if (a.stats) {
+  if (o.stats) {
     // block totals: clipped count and the largest raw nu_t (non-negative, so
     // its bit pattern orders like the value)
     __shared__ uint32_t s_cnt[4], s_max[4];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      cnt += __shfl_xor(cnt, o);
-      mx = max(mx, (uint32_t)__shfl_xor(mx, o));
+    for (int l = 32; l > 0; l >>= 1) {
+      cnt += __shfl_xor(cnt, l);
+      mx = max(mx, (uint32_t)__shfl_xor(mx, l));
     }
     const uint32_t w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
@@ -338,8 +245,8 @@ __global__ __launch_bounds__(256) void k_wale(WaleArgs a) {
     if (threadIdx.x == 0) {
       const uint32_t c = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
       const uint32_t b = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-      if (c) atomicAdd(&a.stats[0], c);
-      if (b) atomicMax(&a.stats[1], b);
+      if (c) atomicAdd(&o.stats[0], c);
+      if (b) atomicMax(&o.stats[1], b);
     }
   }
 }
@@ -359,19 +266,27 @@ static uint32_t wale_zlen(const Dom& d) {
   return z;
 }
 
-template <typename S>
-static hipError_t wale_s(int Q, WaleArgs a, hipStream_t s) {
-  a.zlen = wale_zlen(a.d);
+template <int Q, typename S>
+static void local_q(const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
   const dim3 grid((a.d.N + 255) / 256), block(256);
-  const dim3 tiles((a.d.nx + kWaleTileX - 1) / kWaleTileX, (a.d.ny + kWaleTileY - 1) / kWaleTileY,
-                   (a.d.nz + a.zlen - 1) / a.zlen);
-  if (Q == 19) {
-    hipLaunchKernelGGL((k_wale_local<19, S>), grid, block, 0, s, a);
-    hipLaunchKernelGGL((k_wale<19, S>), tiles, block, 0, s, a);
-  } else {
-    hipLaunchKernelGGL((k_wale_local<27, S>), grid, block, 0, s, a);
-    hipLaunchKernelGGL((k_wale<27, S>), tiles, block, 0, s, a);
-  }
+  const uint32_t deal = a.d.N < (1u << 24) ? kXcdStretch : 5u;
+  const ScalarStepArgs none{};
+  if (sc)
+    hipLaunchKernelGGL((k_wale_local<Q, S, false, 7>), grid, block, 0, s, a, deal, *sc);
+  else if (a.d.per[0] || a.d.per[1] || a.d.per[2] || a.open)
+    hipLaunchKernelGGL((k_wale_local<Q, S, true, 0>), grid, block, 0, s, a, deal, none);
+  else
+    hipLaunchKernelGGL((k_wale_local<Q, S, false, 0>), grid, block, 0, s, a, deal, none);
+}
+
+hipError_t launch_wale_local(int Q, int storage, const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
+  if (a.d.N == 0) return hipSuccess;
+  if (storage == kF32)
+    Q == 19 ? local_q<19, float>(a, sc, s) : local_q<27, float>(a, sc, s);
+  else if (storage == kF16)
+    Q == 19 ? local_q<19, _Float16>(a, sc, s) : local_q<27, _Float16>(a, sc, s);
+  else
+    Q == 19 ? local_q<19, bf16s>(a, sc, s) : local_q<27, bf16s>(a, sc, s);
   return hipGetLastError();
 }
 
@@ -380,21 +295,19 @@ __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
   if (k < n) p[k] = 0u;
 }
 
-hipError_t launch_wale(int Q, int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
-                       const float* wall_u, const float* F_cur, const float* F_mom, float* work, const HydroParams& p,
-                       float tau_eff, float cw_delta_sq, float nu0, float nut_max, float* omega, float* nut,
-                       uint32_t* stats, hipStream_t s) {
-  if (d.N == 0) return hipSuccess;
+hipError_t launch_wale_omega(const WaleFields& a, float cw_delta_sq, float nu0, float nut_max, float* omega,
+                             float* nut, uint32_t* stats, hipStream_t s) {
+  if (a.d.N == 0) return hipSuccess;
   if (stats) {
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, stats, 2u);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  WaleArgs a{d,           f,       mask, wall_u, F_cur, F_mom, p,     odd, tau_eff, cw_delta_sq,
-             nu0,         nut_max, work, work + 3 * (size_t)d.N, omega, nut, stats};
-  if (storage == kF32) return wale_s<float>(Q, a, s);
-  if (storage == kF16) return wale_s<_Float16>(Q, a, s);
-  return wale_s<bf16s>(Q, a, s);
+  const uint32_t zlen = wale_zlen(a.d);
+  const dim3 tiles((a.d.nx + kWaleTileX - 1) / kWaleTileX, (a.d.ny + kWaleTileY - 1) / kWaleTileY,
+                   (a.d.nz + zlen - 1) / zlen);
+  hipLaunchKernelGGL(k_wale, tiles, dim3(256), 0, s, a, WaleOut{cw_delta_sq, nu0, nut_max, omega, nut, stats}, zlen);
+  return hipGetLastError();
 }
 
 }  // namespace lbm

@@ -345,7 +345,7 @@ static void scalar_step_s(int Q, int Qs, const VelArgs& a, const ScalarStepArgs&
 }
 
 // This step's buffers and concentration; the state moves on to the next.
-static int scalar_turn(const FieldsView& v, ScalarState* s, ScalarStepArgs* st) {
+int scalar_turn(const FieldsView& v, ScalarState* s, ScalarStepArgs* st) {
   if (s->dirty2) {
     hipLaunchKernelGGL(k_scalar_zero_solid, dim3(nblk(v.d.N)), dim3(256), 0, v.stream, v.d, v.mask, s->h2, s->ps,
                        s->Qs);

@@ -5,14 +5,6 @@
 
 namespace lbm {
 
-struct ScalarStepArgs {
-  const float* h;   // Qs planes: this step's distribution
-  float* h2;        // Qs planes: the next one
-  const float* C;   // concentration to collide with, null: the sum of h
-  size_t ps;        // plane stride
-  float omega;
-};
-
 // h_eq of scalar_equilibrium (scalar.rs:6-15) for the hydro lattice; the
 // D3Q7 form uses 1/cs^2 = 4.
 template <int Qs, int q>
