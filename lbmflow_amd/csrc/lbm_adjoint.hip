@@ -36,43 +36,59 @@ struct AdjArgs {
   double* omega_bar;     // N: accumulated adjoint of omega_plus
   double* Fbar;          // N x 3: adjoint of F_cur (forced cells; others untouched)
   double* Gout;          // N x 3: adjoint of F_mom (forced cells; others untouched)
+  const uint32_t* flist;  // the force list (forced cells), or none
+  uint32_t nlist;
+  uint32_t deal;
 };
 
-template <typename S, bool ODD>
-__global__ __launch_bounds__(256) void k_adj_collide_stream(AdjArgs a) {
+// Bound by HBM: 2 x 152 bytes of adjoint populations, 76 of populations, 16 of
+// omega_bar per fluid cell.  Per pair of opposite directions everything the
+// transposed Jacobian needs of feq and S is a multiple of Lp = lam*_a + lam*_b
+// and Lm = lam*_a - lam*_b, so the direct part, the feq and the S adjoints are
+// never stored: what lives through the kernel is lam* (19 f64) and f (19 fp32).
+// The form that held all three took 296 VGPRs, one wave per SIMD, and 240 us
+// on the 128^3 tank; this one 168, three waves, and 162 us (0.53 GB, 3.3 TB/s).
+// Solid cells are skipped: no fluid cell reads their adjoint, which stays zero.
+// FORCED cells (those of the force list) take the source's terms as well, in a
+// launch of their own over the list: in one kernel that rare branch sets the
+// register count.
+template <typename S, bool ODD, bool WRAP, bool FORCED>
+__device__ __forceinline__ void adj_cell(const AdjArgs& a, uint32_t i, uint32_t m) {
   constexpr int Q = 19;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.d.N) return;
-  const uint32_t m = a.mask[i];
   const size_t N = a.d.N;
-  if (m & kMaskSolid) {
-    sfor<0, Q>([&](auto qc) { a.lam_out[(size_t)decltype(qc)::value * N + i] = 0.0; });
-    return;
-  }
-  uint32_t x, y, z;
-  cell_xyz(a.d, i, x, y, z);
-  const Nbr nb(a.d, x, y, z);
-  // forward state
-  double f[Q];
-  sfor<0, Q>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    f[q] = (double)read_pop<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, ODD);
-  });
-  // adjoint of the post-collision populations, pulled through the streaming
+  uint32_t x = 0, y = 0, z = 0;
+  if constexpr (WRAP) cell_xyz(a.d, i, x, y, z);
+  const Nbr nb = WRAP ? Nbr(a.d, x, y, z) : Nbr(a.d);
+  // forward state, and the adjoint of the post-collision populations pulled
+  // through the streaming
+  float f[Q];
   double ls[Q];
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    constexpr int o = lat_opp(q);
-    if ((m >> o) & 1u) {
-      ls[q] = a.lam_in[(size_t)o * N + i];
-    } else {
-      const uint32_t j = i + (uint32_t)nb.template off<lat_c(q, 0), lat_c(q, 1), lat_c(q, 2)>();
+    f[q] = read_pop<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, ODD);
+  });
+  // (plane bases are uniform, the per-lane part is one 32-bit byte offset: the
+  // f64 planes of a domain that fits the card stay below 4 GiB)
+  const uint32_t at = i * 8u;
+  sfor<0, Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    constexpr int cx = lat_c(q, 0), cy = lat_c(q, 1), cz = lat_c(q, 2);
+    if constexpr (WRAP) {
+      const uint32_t j = i + (uint32_t)nb.template off<cx, cy, cz>();
       ls[q] = a.lam_in[(size_t)q * N + j];
+    } else {
+      const int64_t shift = cx + cy * (int64_t)a.d.nx + cz * (int64_t)a.d.nx * a.d.ny;
+      ls[q] = *(const double*)((const char*)(a.lam_in + (int64_t)(q * N) + shift) + at);
     }
   });
-  const bool forced = (m & kMaskForced) != 0 && a.F_cur && a.F_mom;
+  if (m & kMaskLinks)  // reflected ones: i + c_q is solid
+    sfor<1, Q>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      constexpr int o = lat_opp(q);
+      if ((m >> o) & 1u) ls[q] = *(const double*)((const char*)(a.lam_in + o * N) + at);
+    });
   double Fm[3] = {0.0, 0.0, 0.0}, Fc[3] = {0.0, 0.0, 0.0};
-  if (forced)
+  if constexpr (FORCED)
     for (int c = 0; c < 3; ++c) {
       Fm[c] = (double)a.F_mom[3 * (size_t)i + c];
       Fc[c] = (double)a.F_cur[3 * (size_t)i + c];
@@ -81,109 +97,192 @@ __global__ __launch_bounds__(256) void k_adj_collide_stream(AdjArgs a) {
   const double cp = 1.0 - 0.5 * op;
   const double om = (double)a.p.omega_m, cm = (double)a.p.cm;
   // moments
-  double r = 1.0, mv[3] = {0.0, 0.0, 0.0};
+  double r = 1.0, u[3] = {0.0, 0.0, 0.0};
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    r += f[q];
-    if constexpr (lat_c(q, 0) != 0) mv[0] += (double)lat_c(q, 0) * f[q];
-    if constexpr (lat_c(q, 1) != 0) mv[1] += (double)lat_c(q, 1) * f[q];
-    if constexpr (lat_c(q, 2) != 0) mv[2] += (double)lat_c(q, 2) * f[q];
+    const double fq = (double)f[q];
+    r += fq;
+    if constexpr (lat_c(q, 0) != 0) u[0] += (double)lat_c(q, 0) * fq;
+    if constexpr (lat_c(q, 1) != 0) u[1] += (double)lat_c(q, 1) * fq;
+    if constexpr (lat_c(q, 2) != 0) u[2] += (double)lat_c(q, 2) * fq;
   });
-  const double u[3] = {(mv[0] + 0.5 * Fm[0]) / r, (mv[1] + 0.5 * Fm[1]) / r, (mv[2] + 0.5 * Fm[2]) / r};
+  for (int c = 0; c < 3; ++c) u[c] = (u[c] + 0.5 * Fm[c]) / r;
   const double usq = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
   const double uf = u[0] * Fc[0] + u[1] * Fc[1] + u[2] * Fc[2];
-  double lo[Q], eb[Q], sb[Q];  // adjoint of f (direct part), of feq, of S
-  double obar = 0.0;
-  auto feq = [&](double cu, double w) { return w * (r - 1.0 + r * (3.0 * cu + 4.5 * cu * cu - 1.5 * usq)); };
-  auto src = [&](double cu, double cf, double w) { return w * (3.0 * (cf - uf) + 9.0 * cu * cf); };
-  {  // rest population
-    const double w0 = (double)lat_wf(Q, 0);
-    const double e0 = feq(0.0, w0), s0 = forced ? src(0.0, 0.0, w0) : 0.0;
-    lo[0] = ls[0] * (1.0 - op);
-    eb[0] = ls[0] * op;
-    sb[0] = ls[0] * cp;
-    obar += ls[0] * (-(f[0] - e0) - 0.5 * s0);
-  }
+  // feq back to rho and u: with eb_a +- eb_b = op Lp, om Lm,
+  //   rho: w (op Lp (1 + 4.5 cu^2 - 1.5 u.u) + om Lm 3 cu)
+  //   u:   w r (op Lp (9 cu c - 3 u) + 3 om Lm c)
+  const double w0 = (double)lat_wf(Q, 0);
+  const double sym = 1.0 - 1.5 * usq;
+  double rb = op * ls[0] * w0 * sym;
+  double lpw = op * ls[0] * w0;  // sum w op Lp: the -3 u part of the u adjoint
+  double ub[3] = {0.0, 0.0, 0.0};
+  double obar = ls[0] * -((double)f[0] - w0 * (r - 1.0 - r * 1.5 * usq));
   sfor<0, (Q - 1) / 2>([&](auto kc) {
     constexpr int qa = 2 * decltype(kc)::value + 1;
     constexpr int qb = qa + 1;
     const double w = (double)lat_wf(Q, qa);
-    const double cua = (double)lat_c(qa, 0) * u[0] + (double)lat_c(qa, 1) * u[1] + (double)lat_c(qa, 2) * u[2];
-    const double cub = -cua;
-    const double ea = feq(cua, w), ebb = feq(cub, w);
-    double sa = 0.0, sbb = 0.0;
-    if (forced) {
-      const double cfa = (double)lat_c(qa, 0) * Fc[0] + (double)lat_c(qa, 1) * Fc[1] + (double)lat_c(qa, 2) * Fc[2];
-      sa = src(cua, cfa, w);
-      sbb = src(cub, -cfa, w);
-    }
-    const double Lp = ls[qa] + ls[qb], Lm = ls[qa] - ls[qb];
-    lo[qa] = ls[qa] - 0.5 * op * Lp - 0.5 * om * Lm;
-    lo[qb] = ls[qb] - 0.5 * op * Lp + 0.5 * om * Lm;
-    eb[qa] = 0.5 * op * Lp + 0.5 * om * Lm;
-    eb[qb] = 0.5 * op * Lp - 0.5 * om * Lm;
-    sb[qa] = 0.5 * cp * Lp + 0.5 * cm * Lm;
-    sb[qb] = 0.5 * cp * Lp - 0.5 * cm * Lm;
-    const double fp = 0.5 * (f[qa] + f[qb]), ep = 0.5 * (ea + ebb), sp = 0.5 * (sa + sbb);
-    obar += Lp * (-(fp - ep) - 0.5 * sp);
+    double cu = 0.0;
+    if constexpr (lat_c(qa, 0) != 0) cu += (double)lat_c(qa, 0) * u[0];
+    if constexpr (lat_c(qa, 1) != 0) cu += (double)lat_c(qa, 1) * u[1];
+    if constexpr (lat_c(qa, 2) != 0) cu += (double)lat_c(qa, 2) * u[2];
+    const double Lp = ls[qa] + ls[qb];
+    const double P = w * op * Lp, M = w * om * (ls[qa] - ls[qb]);
+    const double cu2 = 4.5 * cu * cu;
+    rb += P * (sym + cu2) + M * (3.0 * cu);
+    lpw += P;
+    const double t = P * (9.0 * cu) + 3.0 * M;
+    if constexpr (lat_c(qa, 0) != 0) ub[0] += (double)lat_c(qa, 0) * t;
+    if constexpr (lat_c(qa, 1) != 0) ub[1] += (double)lat_c(qa, 1) * t;
+    if constexpr (lat_c(qa, 2) != 0) ub[2] += (double)lat_c(qa, 2) * t;
+    const double ep = w * (r - 1.0 + r * (cu2 - 1.5 * usq));
+    obar -= Lp * (0.5 * ((double)f[qa] + (double)f[qb]) - ep);
   });
-  // feq and S back to rho, u, F_cur
-  double rb = 0.0, ub[3] = {0.0, 0.0, 0.0}, fcb[3] = {0.0, 0.0, 0.0};
-  sfor<0, Q>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    const double w = (double)lat_wf(Q, q);
-    const double c[3] = {(double)lat_c(q, 0), (double)lat_c(q, 1), (double)lat_c(q, 2)};
-    const double cu = c[0] * u[0] + c[1] * u[1] + c[2] * u[2];
-    rb += eb[q] * w * (1.0 + 3.0 * cu + 4.5 * cu * cu - 1.5 * usq);
-    for (int al = 0; al < 3; ++al) ub[al] += eb[q] * w * r * (3.0 * c[al] + 9.0 * cu * c[al] - 3.0 * u[al]);
-    if (forced) {
-      const double cf = c[0] * Fc[0] + c[1] * Fc[1] + c[2] * Fc[2];
-      for (int al = 0; al < 3; ++al) {
-        ub[al] += sb[q] * w * (-3.0 * Fc[al] + 9.0 * c[al] * cf);
-        fcb[al] += sb[q] * w * (3.0 * (c[al] - u[al]) + 9.0 * cu * c[al]);
+  for (int c = 0; c < 3; ++c) ub[c] = r * (ub[c] - 3.0 * lpw * u[c]);
+  // Each phase recomputes its pair sums from lam*: kept from one phase to the
+  // next (as the compiler would) they cost 54 registers.
+  auto fresh = [](double* v) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(v[q]));
+  };
+  fresh(ls);
+  if constexpr (FORCED) {
+    // the source back to u and F_cur, and its share of omega_bar: with
+    // sb_a +- sb_b = cp Lp, cm Lm
+    double fcb[3] = {0.0, 0.0, 0.0};
+    const double s0 = cp * ls[0] * w0;
+    obar += ls[0] * -0.5 * (w0 * (-3.0 * uf));
+    for (int c = 0; c < 3; ++c) {
+      ub[c] += -3.0 * s0 * Fc[c];
+      fcb[c] += -3.0 * s0 * u[c];
+    }
+    sfor<0, (Q - 1) / 2>([&](auto kc) {
+      constexpr int qa = 2 * decltype(kc)::value + 1;
+      constexpr int qb = qa + 1;
+      const double w = (double)lat_wf(Q, qa);
+      const double c3[3] = {(double)lat_c(qa, 0), (double)lat_c(qa, 1), (double)lat_c(qa, 2)};
+      const double cu = c3[0] * u[0] + c3[1] * u[1] + c3[2] * u[2];
+      const double cf = c3[0] * Fc[0] + c3[1] * Fc[1] + c3[2] * Fc[2];
+      const double Lp = ls[qa] + ls[qb];
+      const double P = w * cp * Lp, M = w * cm * (ls[qa] - ls[qb]);
+      for (int c = 0; c < 3; ++c) {
+        ub[c] += P * (-3.0 * Fc[c] + 9.0 * c3[c] * cf);
+        fcb[c] += P * (-3.0 * u[c] + 9.0 * cu * c3[c]) + 3.0 * M * c3[c];
       }
+      obar -= 0.5 * Lp * (w * (-3.0 * uf + 9.0 * cu * cf));
+    });
+    for (int c = 0; c < 3; ++c) {
+      a.Fbar[3 * (size_t)i + c] = fcb[c];
+      a.Gout[3 * (size_t)i + c] = ub[c] / (2.0 * r);
     }
-  });
+  }
   // u = (m + F_mom/2)/rho
   double mb[3];
-  for (int al = 0; al < 3; ++al) {
-    mb[al] = ub[al] / r;
-    rb += -ub[al] * u[al] / r;
+  for (int c = 0; c < 3; ++c) {
+    mb[c] = ub[c] / r;
+    rb += -ub[c] * u[c] / r;
   }
-  sfor<0, Q>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    double v = lo[q] + rb;
-    if constexpr (lat_c(q, 0) != 0) v += (double)lat_c(q, 0) * mb[0];
-    if constexpr (lat_c(q, 1) != 0) v += (double)lat_c(q, 1) * mb[1];
-    if constexpr (lat_c(q, 2) != 0) v += (double)lat_c(q, 2) * mb[2];
-    a.lam_out[(size_t)q * N + i] = v;
+  fresh(ls);
+  auto out = [&](int q) { return (double*)((char*)(a.lam_out + (size_t)q * N) + at); };
+  *out(0) = ls[0] * (1.0 - op) + rb;
+  sfor<0, (Q - 1) / 2>([&](auto kc) {
+    constexpr int qa = 2 * decltype(kc)::value + 1;
+    constexpr int qb = qa + 1;
+    const double ep = 0.5 * op * (ls[qa] + ls[qb]), em = 0.5 * om * (ls[qa] - ls[qb]);
+    double cmb = 0.0;
+    if constexpr (lat_c(qa, 0) != 0) cmb += (double)lat_c(qa, 0) * mb[0];
+    if constexpr (lat_c(qa, 1) != 0) cmb += (double)lat_c(qa, 1) * mb[1];
+    if constexpr (lat_c(qa, 2) != 0) cmb += (double)lat_c(qa, 2) * mb[2];
+    *out(qa) = ls[qa] - ep - em + rb + cmb;
+    *out(qb) = ls[qb] - ep + em + rb - cmb;
   });
   a.omega_bar[i] += obar;
-  if (forced)
-    for (int al = 0; al < 3; ++al) {
-      a.Fbar[3 * (size_t)i + al] = fcb[al];
-      a.Gout[3 * (size_t)i + al] = ub[al] / (2.0 * r);
-    }
+}
+
+template <typename S, bool ODD, bool WRAP>
+__global__ __launch_bounds__(256, 3) void k_adj_collide_stream(AdjArgs a) {
+  const uint32_t i = xcd_remap(blockIdx.x, gridDim.x, a.deal) * 256 + threadIdx.x;
+  if (i >= a.d.N) return;
+  const uint32_t m = a.mask[i];
+  if ((m & kMaskSolid) || (a.nlist && (m & kMaskForced))) return;
+  adj_cell<S, ODD, WRAP, false>(a, i, m);
+}
+
+template <typename S, bool ODD>
+__global__ __launch_bounds__(64) void k_adj_list(AdjArgs a) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= a.nlist) return;
+  const uint32_t i = a.flist[k];
+  const uint32_t m = a.mask[i];
+  if (!(m & kMaskSolid)) adj_cell<S, ODD, true, true>(a, i, m);
 }
 
 template <typename S>
 static hipError_t adj_s(int odd, const AdjArgs& a, hipStream_t s) {
   const dim3 grid((a.d.N + 255) / 256), block(256);
-  if (odd)
-    hipLaunchKernelGGL((k_adj_collide_stream<S, true>), grid, block, 0, s, a);
+  const bool wrap = a.d.per[0] || a.d.per[1] || a.d.per[2];
+  if (odd && wrap)
+    hipLaunchKernelGGL((k_adj_collide_stream<S, true, true>), grid, block, 0, s, a);
+  else if (odd)
+    hipLaunchKernelGGL((k_adj_collide_stream<S, true, false>), grid, block, 0, s, a);
+  else if (wrap)
+    hipLaunchKernelGGL((k_adj_collide_stream<S, false, true>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((k_adj_collide_stream<S, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_adj_collide_stream<S, false, false>), grid, block, 0, s, a);
+  if (a.nlist) {
+    const dim3 lg((a.nlist + 63) / 64), lb(64);
+    if (odd)
+      hipLaunchKernelGGL((k_adj_list<S, true>), lg, lb, 0, s, a);
+    else
+      hipLaunchKernelGGL((k_adj_list<S, false>), lg, lb, 0, s, a);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_adj_collide_stream(int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
                                      const float* omega, const float* F_cur, const float* F_mom,
-                                     const HydroParams& p, const double* lam_in, double* lam_out, double* omega_bar,
-                                     double* Fbar, double* Gout, hipStream_t s) {
-  AdjArgs a{d, f, mask, omega, F_cur, F_mom, p, lam_in, lam_out, omega_bar, Fbar, Gout};
+                                     const HydroParams& p, const uint32_t* flist, uint32_t nlist, const double* lam_in,
+                                     double* lam_out, double* omega_bar, double* Fbar, double* Gout,
+                                     hipStream_t s) {
+  AdjArgs a{d, f, mask, omega, F_cur, F_mom, p, lam_in, lam_out, omega_bar, Fbar, Gout,
+            flist, F_cur && F_mom ? nlist : 0u, 5u};
   if (storage == kF32) return adj_s<float>(odd, a, s);
   if (storage == kF16) return adj_s<_Float16>(odd, a, s);
   return adj_s<bf16s>(odd, a, s);
+}
+
+// dJ/dnu from the adjoint of omega_plus = 1 / (3 nu + 1/2): times -3 omega_plus^2
+__global__ void k_nu_bar(uint32_t n, const double* omega_bar, const float* omega, float omega_p, double* out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double op = omega ? (double)omega[i] : (double)omega_p;
+  out[i] = omega_bar[i] * (-3.0 * op * op);
+}
+
+// the listed cells' vec3 of F into buf (dir 0) or back (dir 1)
+__global__ void k_list_pack(const uint32_t* flist, uint32_t n, float* F, float* buf, int dir) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const size_t i = flist[k];
+  for (int c = 0; c < 3; ++c) {
+    if (dir == 0)
+      buf[3 * (size_t)k + c] = F[3 * i + c];
+    else
+      F[3 * i + c] = buf[3 * (size_t)k + c];
+  }
+}
+
+hipError_t launch_list_pack(const uint32_t* flist, uint32_t n, float* F, float* buf, int dir, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_list_pack, dim3((n + 255) / 256), dim3(256), 0, s, flist, n, F, buf, dir);
+  return hipGetLastError();
+}
+
+hipError_t launch_nu_bar(uint32_t n, const double* omega_bar, const float* omega, float omega_p, double* out,
+                         hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_nu_bar, dim3((n + 255) / 256), dim3(256), 0, s, n, omega_bar, omega, omega_p, out);
+  return hipGetLastError();
 }
 
 __global__ void k_fill_d(double* p, size_t n, double v) {

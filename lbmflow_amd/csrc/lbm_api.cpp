@@ -2571,6 +2571,8 @@ void revolve(int lo, int hi, int slot, int free_slots, std::vector<int>& out) {
   }
 }
 
+// One saved state: the population buffer, the cached-moment force at the
+// listed cells (it is zero elsewhere), the parity and the clock.
 struct Snapshot {
   void* f = nullptr;
   float* F_mom = nullptr;
@@ -2580,10 +2582,8 @@ struct Snapshot {
 
 int snap_save(lbm_fields* fl, Snapshot& sn) {
   hipStream_t s = fl->ctx->stream;
-  if (!sn.f) HIPCHK(fl->ctx, hipMalloc(&sn.f, fl->f_bytes));
-  if (!sn.F_mom) HIPCHK(fl->ctx, hipMalloc((void**)&sn.F_mom, N3(fl) * 4));
   HIPCHK(fl->ctx, hipMemcpyAsync(sn.f, fl->f_alloc, fl->f_bytes, hipMemcpyDeviceToDevice, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(sn.F_mom, fl->F_mom, N3(fl) * 4, hipMemcpyDeviceToDevice, s));
+  HIPCHK(fl->ctx, launch_list_pack(fl->flist, (uint32_t)fl->flist_host.size(), fl->F_mom, sn.F_mom, 0, s));
   sn.parity = fl->parity;
   sn.time = fl->time;
   return LBM_OK;
@@ -2592,16 +2592,10 @@ int snap_save(lbm_fields* fl, Snapshot& sn) {
 int snap_restore(lbm_fields* fl, const Snapshot& sn) {
   hipStream_t s = fl->ctx->stream;
   HIPCHK(fl->ctx, hipMemcpyAsync(fl->f_alloc, sn.f, fl->f_bytes, hipMemcpyDeviceToDevice, s));
-  HIPCHK(fl->ctx, hipMemcpyAsync(fl->F_mom, sn.F_mom, N3(fl) * 4, hipMemcpyDeviceToDevice, s));
+  HIPCHK(fl->ctx, launch_list_pack(fl->flist, (uint32_t)fl->flist_host.size(), fl->F_mom, sn.F_mom, 1, s));
   fl->parity = sn.parity;
   fl->time = sn.time;
   return LBM_OK;
-}
-
-void snap_free(Snapshot& sn) {
-  if (sn.f) (void)hipFree(sn.f);
-  if (sn.F_mom) (void)hipFree(sn.F_mom);
-  sn = Snapshot{};
 }
 
 }  // namespace
@@ -2645,22 +2639,32 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     rc = ibm_set_domains(view_of(fl), fl->ibm, &D);
     if (rc) return rc;
   }
-  std::vector<Snapshot> snap((size_t)snapshots + 1);
+  const bool gradients = dJ_domega || dJ_dnu;
+  // The schedule tells how many slots it fills; those, the final state and the
+  // adjoint arrays are one allocation (17 of them with their frees took 10 ms of
+  // a 46 ms call at 128^3 with 8 snapshots).
+  std::vector<int> plan;
+  size_t slots = 0;
+  if (gradients) {
+    revolve(0, steps, 0, snapshots, plan);
+    slots = 1;
+    for (size_t k = 0; k < plan.size(); k += 2)
+      if (plan[k] == ACT_SAVE) slots = std::max(slots, (size_t)plan[k + 1] + 1);
+  }
+  std::vector<Snapshot> snap(slots);
   Snapshot fin;
   double *lamA = nullptr, *lamB = nullptr, *obar = nullptr, *Fbar = nullptr, *G0 = nullptr, *G1 = nullptr,
          *wbar = nullptr;
+  char* slab = nullptr;
   // a failure after the forward pass puts the final state back (best
-  // effort) before every snapshot and adjoint buffer is freed
+  // effort) before the allocation is freed
   bool reversing = false;
   auto cleanup = [&]() {
     const std::string err = fl->ctx->err;  // the failure being reported
-    if (reversing && fin.f) (void)snap_restore(fl, fin);
+    if (reversing) (void)snap_restore(fl, fin);
     (void)hipStreamSynchronize(s);
     fl->ctx->err = err;
-    for (Snapshot& sn : snap) snap_free(sn);
-    snap_free(fin);
-    for (double* p : {lamA, lamB, obar, Fbar, G0, G1, wbar})
-      if (p) (void)hipFree(p);
+    if (slab) (void)hipFree(slab);
   };
   auto hip_rc = [&](hipError_t e, const char* what) -> int {
     return e == hipSuccess ? LBM_OK : fail(fl->ctx, LBM_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
@@ -2674,35 +2678,51 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     }                   \
   } while (0)
 #define ADJ_HIP(expr) ADJ_TRY(hip_rc((expr), #expr))
+  if (gradients) {
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t fb = up(fl->f_bytes), lb = up(3 * sizeof(float) * std::max<size_t>(1, fl->flist_host.size()));
+    // zeroed: lamA, the force adjoints, omega_bar, the rotation rate's
+    const size_t nz = Q * N + 9 * N + N + 1;
+    const size_t bytes = (slots + 1) * (fb + lb) + up(nz * sizeof(double)) + Q * N * sizeof(double);
+    if (hipMalloc((void**)&slab, bytes) != hipSuccess) {
+      slab = nullptr;
+      return fail(fl->ctx, LBM_ERR_NOMEM, "adjoint workspace of %zu bytes (%zu snapshots)", bytes, slots + 1);
+    }
+    char* at = slab;
+    auto take = [&](size_t b) {
+      char* p = at;
+      at += b;
+      return p;
+    };
+    for (Snapshot& sn : snap) {
+      sn.f = take(fb);
+      sn.F_mom = (float*)take(lb);
+    }
+    fin.f = take(fb);
+    fin.F_mom = (float*)take(lb);
+    lamA = (double*)take(up(nz * sizeof(double)));
+    lamB = (double*)take(Q * N * sizeof(double));
+    G0 = lamA + Q * N;
+    G1 = G0 + 3 * N;
+    Fbar = G1 + 3 * N;
+    wbar = Fbar + 3 * N;
+    obar = wbar + N;
+    ADJ_HIP(launch_fill_f64(lamA, nz, 0.0, s));
+    ADJ_TRY(snap_save(fl, snap[0]));
+  }
   // forward pass: J
-  ADJ_TRY(snap_save(fl, snap[0]));
   std::vector<double> tq(3 * (size_t)steps);
   ADJ_TRY(lbm_run_ibm_span(fl, steps, 0, tq.data(), nullptr));
   double acc = 0.0;
   for (int k = steps - window; k < steps; ++k) acc += -tq[3 * (size_t)k + 2];
   *J = acc / window;
-  ADJ_TRY(snap_save(fl, fin));
-  if (!dJ_domega && !dJ_dnu) {
+  if (!gradients) {
     cleanup();
     return LBM_OK;
   }
+  ADJ_TRY(snap_save(fl, fin));
   // reverse pass
   reversing = true;
-  auto dalloc = [&](double** p, size_t n) -> int {
-    if (hipMalloc((void**)p, n * sizeof(double)) != hipSuccess)
-      return fail(fl->ctx, LBM_ERR_NOMEM, "adjoint buffer of %zu doubles", n);
-    HIPCHK(fl->ctx, launch_fill_f64(*p, n, 0.0, s));
-    return LBM_OK;
-  };
-  ADJ_TRY(dalloc(&lamA, Q * N));
-  ADJ_TRY(dalloc(&lamB, Q * N));
-  ADJ_TRY(dalloc(&obar, 1));
-  ADJ_TRY(dalloc(&Fbar, 3 * N));
-  ADJ_TRY(dalloc(&G0, 3 * N));
-  ADJ_TRY(dalloc(&G1, 3 * N));
-  ADJ_TRY(dalloc(&wbar, N));
-  std::vector<int> plan;
-  revolve(0, steps, 0, snapshots, plan);
   int64_t advanced = steps;
   const double tq_bar = 1.0 / window;
   // the snapshot slot the device state still equals (the schedule restores
@@ -2728,27 +2748,22 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
       ADJ_TRY(ibm_enqueue_recorded(view_of(fl), fl->ibm));
       fl->field_present = true;
       ADJ_HIP(launch_adj_collide_stream(fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->omega,
-                                                fl->F_cur, fl->F_mom, fl->hp, lamA, lamB, wbar, Fbar, G1, s));
+                                                fl->F_cur, fl->F_mom, fl->hp, fl->flist,
+                                        (uint32_t)fl->flist_host.size(), lamA, lamB, wbar, Fbar, G1, s));
       ADJ_TRY(ibm_adjoint(view_of(fl), fl->ibm, Fbar, G0, arg >= steps - window ? tq_bar : 0.0, lamB, obar));
       std::swap(lamA, lamB);
       std::swap(G0, G1);
     }
   }
   double ob = 0.0;
-  std::vector<double> wb(dJ_dnu ? N : 0);
   ADJ_HIP(hipMemcpyAsync(&ob, obar, sizeof ob, hipMemcpyDeviceToHost, s));
-  if (dJ_dnu) ADJ_HIP(hipMemcpyAsync(wb.data(), wbar, N * sizeof(double), hipMemcpyDeviceToHost, s));
-  std::vector<float> om(fl->omega && dJ_dnu ? N : 0);
-  if (!om.empty()) ADJ_HIP(hipMemcpyAsync(om.data(), fl->omega, N * 4, hipMemcpyDeviceToHost, s));
-  ADJ_HIP(hipStreamSynchronize(s));
-  if (dJ_domega) *dJ_domega = ob;
   if (dJ_dnu) {
     // omega_plus = 1 / (3 nu + 1/2): d omega_plus / d nu = -3 omega_plus^2
-    for (size_t i = 0; i < N; ++i) {
-      const double op = om.empty() ? (double)fl->hp.omega_p : (double)om[i];
-      dJ_dnu[i] = wb[i] * (-3.0 * op * op);
-    }
+    ADJ_HIP(launch_nu_bar((uint32_t)N, wbar, fl->omega, fl->hp.omega_p, lamB, s));
+    ADJ_TRY(read_array(fl, dJ_dnu, lamB, N * sizeof(double)));
   }
+  ADJ_HIP(hipStreamSynchronize(s));
+  if (dJ_domega) *dJ_domega = ob;
   if (forward_steps) *forward_steps = advanced;
   ADJ_TRY(snap_restore(fl, fin));
   ADJ_TRY(finish_scalars(fl));

@@ -212,8 +212,14 @@ hipError_t launch_clear_batch(const HydroArgs* tab, const uint32_t* cells, uint3
 // Adjoint of one D3Q19 TRT/BGK collide-stream step (lbm_adjoint.hip).
 hipError_t launch_adj_collide_stream(int storage, int odd, const Dom& d, const void* f, const uint32_t* mask,
                                      const float* omega, const float* F_cur, const float* F_mom,
-                                     const HydroParams& p, const double* lam_in, double* lam_out, double* omega_bar,
-                                     double* Fbar, double* Gout, hipStream_t s);
+                                     const HydroParams& p, const uint32_t* flist, uint32_t nlist, const double* lam_in,
+                                     double* lam_out, double* omega_bar, double* Fbar, double* Gout,
+                                     hipStream_t s);
+// the listed cells' vec3 of F into buf (dir 0) or back (dir 1)
+hipError_t launch_list_pack(const uint32_t* flist, uint32_t n, float* F, float* buf, int dir, hipStream_t s);
+// dJ/dnu of n cells from the adjoint of their omega_plus (omega null: omega_p)
+hipError_t launch_nu_bar(uint32_t n, const double* omega_bar, const float* omega, float omega_p, double* out,
+                         hipStream_t s);
 hipError_t launch_fill_f64(double* p, size_t n, double v, hipStream_t s);
 // probe passes (lbm_probe.hip): post = 0 before the step (densities), 1 after
 hipError_t launch_probe(int Q, int storage, int post, const ProbeArgs& a, hipStream_t s);

@@ -1,0 +1,60 @@
+"""The adjoint collide-stream kernel over the forms it accepts: periodic axes,
+16-bit storage, BGK, obstacles with walls on every side and forced cells in
+wall-linked places, against finite differences of J with respect to the
+per-cell viscosity (the test of test_gpu_adjoint at other domains)."""
+import numpy as np
+import pytest
+
+import lbmflow_amd as L
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("collision,periodic,dims", [("trt", (1, 0, 0), (21, 15, 13)), ("bgk", (0, 0, 0), (18, 17, 13)),
+                                                     ("trt", (1, 1, 1), (16, 12, 9))])
+def test_directional_gradient_matches_differences(collision, periodic, dims):
+    nx, ny, nz = dims
+    solid = np.zeros((nz, ny, nx), np.uint8)
+    for ax, p in enumerate(periodic):
+        if not p:
+            ix = [slice(None)] * 3
+            for k in (0, -1):
+                ix[2 - ax] = k
+                solid[tuple(ix)] = 1
+    solid[3:6, 4:6, 5:7] = 1  # beside the body: forced cells carry wall links
+    rng = np.random.RandomState(2)
+    c = np.array([nx / 2.0, ny / 2.0, nz / 2.0])
+    pos = c + rng.uniform(-3.0, 3.0, (30, 3))
+    n, steps, window, nu0, om = nx * ny * nz, 24, 9, 0.05, 0.012
+    w = 0.3 * np.ones(30)
+
+    def solver(nu):
+        s = L.Solver(19, dims, nu=nu0, collision=collision, periodic=periodic, solid=solid.reshape(-1))
+        s.set_omega_field((1.0 / (3.0 * nu + 0.5)).astype(np.float32))
+        s.set_rotating_body(pos, w, c, (0.0, 0.0, om))
+        return s
+
+    def J(nu):
+        s = solver(nu)
+        v = s.adjoint_torque(steps, window, 0, gradients=False)["J"]
+        s.close()
+        return v
+
+    nu = np.full(n, nu0)
+    s = solver(nu)
+    a = s.adjoint_torque(steps, window, 3)
+    s.close()
+    s = solver(nu)
+    b = s.adjoint_torque(steps, window, 24)
+    s.close()
+    assert a["J"] == b["J"] and np.array_equal(a["dJ_dnu"], b["dJ_dnu"])
+    assert np.all(a["dJ_dnu"][solid.reshape(-1) != 0] == 0.0)
+    x, y, z = cases.coords(dims)
+    d = nu0 * np.cos(2 * np.pi * (x + 2 * y) / nx) * (solid.reshape(-1) == 0)
+    eps = 2e-2
+    diff = [(J(nu + e * d) - J(nu - e * d)) / (2 * e) for e in (eps, 0.5 * eps)]
+    fd = (4.0 * diff[1] - diff[0]) / 3.0  # the second-order error cancels
+    ad = float(np.dot(a["dJ_dnu"], d))
+    # fp32 forward: J carries about 1e-7 of rounding against steps of 1e-2
+    assert abs(ad - fd) <= 2e-3 * abs(fd) + 1e-5 * abs(a["J"])
