@@ -282,14 +282,19 @@ int grow_force_list(lbm_fields* fl, const std::vector<uint32_t>& extra) {
 }
 
 // Rebuild the list of 64-cell tiles the main kernel must visit.  Row tiles
-// are x-segments of one row; when no axis wraps and the row length is not
-// a multiple of 64, tiles are 64-cell blocks of the linear index instead
-// (rows packed end to end: on the 64-tank sweep, edges 48 to 160, 14 %
-// fewer tiles for the same cells), which is exact because without wrapping
-// every neighbour shift is the linear one.
+// are x-segments of one row; when the row length is not a multiple of 64,
+// tiles are 64-cell blocks of the linear index instead (rows packed end to
+// end: on the 64-tank sweep, edges 48 to 160, 14 % fewer tiles for the same
+// cells).  Without wrapping every neighbour shift is the linear one.
 int rebuild_tiles(lbm_fields* fl) {
   const uint32_t nseg = (fl->d.nx + 63) / 64;
-  const bool linear = fl->d.nx % 64 != 0 && !fl->d.per[0] && !fl->d.per[1] && !fl->d.per[2] && !fl->open_face_cells &&
+  const bool wraps = fl->d.per[0] || fl->d.per[1] || fl->d.per[2] || fl->open_face_cells;
+  // Where offsets wrap a linear tile's lanes have to find their coordinates
+  // (two integer divisions), so it is taken when row tiles would leave an
+  // eighth of the lanes idle (periodic 201 x 147 x 173, 21 % idle, even / odd:
+  // D3Q27 bf16 with force 0.170 / 0.199 -> 0.139 / 0.169 ms, fp16 0.128 / 0.167
+  // -> 0.102 / 0.130, fp32 0.211 / 0.245 -> 0.195 / 0.227).
+  const bool linear = fl->d.nx % 64 != 0 && (!wraps || nseg * 64 - fl->d.nx > nseg * 8) &&
                       !(getenv("LBM_ROW_TILES") && getenv("LBM_ROW_TILES")[0] == '1');
   const size_t nt = linear ? ((size_t)fl->d.N + 63) / 64 : (size_t)nseg * fl->d.ny * fl->d.nz;
   uint8_t* dflags = nullptr;

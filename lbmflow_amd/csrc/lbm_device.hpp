@@ -71,9 +71,8 @@ struct Store<bf16s> {
     return __uint_as_float((uint32_t)p[i].v << 16);
   }
   __device__ __forceinline__ static void st(bf16s* p, uint32_t i, float v) {
-    uint32_t b = __float_as_uint(v);
-    b += 0x7FFFu + ((b >> 16) & 1u);  // round to nearest even (finite values)
-    p[i].v = (uint16_t)(b >> 16);
+    // round to nearest even: gfx950's own conversion
+    p[i].v = __builtin_bit_cast(uint16_t, (__bf16)v);
   }
 };
 

@@ -39,10 +39,9 @@ namespace lbm {
 // equilibrium of SecondOrderEq::feq (81-102) and GuoForcing::source
 // (104-121).  Same operand order, no contraction.
 // ---------------------------------------------------------------------------
-template <int Q>
+template <int Q, bool HALVE>
 __device__ __forceinline__ void collide_trt(float* fv, float r, float ux, float uy, float uz, const float Fc[3],
                                             bool fon, float op, float cp, const HydroParams& p) {
-  const float half = 0.5f;
   float usq = ux * ux;
   usq = usq + uy * uy;
   usq = usq + uz * uz;
@@ -54,63 +53,53 @@ __device__ __forceinline__ void collide_trt(float* fv, float r, float ux, float 
   }
   const float drho = r - 1.0f;
   const float f15_usq = 1.5f * usq;
-  auto feq_of = [&](float cu, float w) {
-    float three_cu = 3.0f * cu;
-    float f45_cu = 4.5f * cu;
-    float f45_cu2 = f45_cu * cu;
-    float sum = three_cu + f45_cu2;
-    float inner = sum - f15_usq;
-    float rho_inner = r * inner;
-    float body = drho + rho_inner;
-    return w * body;
-  };
-  auto src_of = [&](float cu, float cf, float w) {
-    float cf_minus_uf = cf - uf;
-    float first = 3.0f * cf_minus_uf;
-    float nine_cu = 9.0f * cu;
-    float second = nine_cu * cf;
-    float body = first + second;
-    return w * body;
-  };
   // rest population
   {
-    const float w0 = lat_wf(Q, 0);
-    float feq0 = feq_of(0.0f * ux, w0);  // cu of the rest velocity is a signed zero
+    constexpr float w0 = lat_wf(Q, 0);
+    const float cu0 = 0.0f * ux;  // cu of the rest velocity is a signed zero
+    const float feq0 = w0 * (drho + r * ((3.0f * cu0 + (4.5f * cu0) * cu0) - f15_usq));
     float f0 = fv[0];
     float relaxed = f0 - op * (f0 - feq0);
     if (fon) {
-      float cf0 = 0.0f;
-      float src0 = src_of(0.0f, cf0, w0);
+      const float src0 = w0 * (3.0f * (0.0f - uf) + (9.0f * cu0) * 0.0f);
       relaxed = relaxed + cp * src0;
     }
     fv[0] = relaxed;
   }
-  const float om = p.omega_m, cm = p.cm;
-  // pairs (q, q+1), q odd, ascending (lattice.rs PAIRS)
+  // Pairs (q, q+1), q odd, ascending (lattice.rs PAIRS).  Every value is the
+  // reference's: cu of the opposite direction is -cu, so the even products are
+  // shared and the odd ones change sign.  HALVE (fp32 storage) halves the pair
+  // sums where the reference does; without it the factor 1/2 goes into the
+  // rates, op (f+ - feq+) = (op/2) ((f_a + f_b) - (e_a + e_b)), the same bits
+  // short of the denormal range, which a front running into fluid at rest does
+  // reach in fp32.  VALU instructions per wave, D3Q19 fp32 486 -> 462, D3Q27
+  // bf16 with force 1158 -> 1000, which is time where 16-bit storage is
+  // VALU-bound (201 x 147 x 173 periodic D3Q27 bf16 with a force, even / odd:
+  // 0.189 / 0.221 -> 0.170 / 0.199 ms with the hardware's bf16 rounding).
+  const float hop = HALVE ? op : 0.5f * op, hom = HALVE ? p.omega_m : 0.5f * p.omega_m;
+  const float hcp = HALVE ? cp : 0.5f * cp, hcm = HALVE ? p.cm : 0.5f * p.cm;
+  auto halve = [](float v) { return HALVE ? 0.5f * v : v; };
   sfor<0, (Q - 1) / 2>([&](auto kc) {
     constexpr int qa = 2 * decltype(kc)::value + 1;
     constexpr int qb = qa + 1;
     constexpr float w = lat_wf(Q, qa);
-    const float cua = cdot<qa>(ux, uy, uz);
-    const float cub = cdot<qb>(ux, uy, uz);
-    const float ea = feq_of(cua, w);
-    const float eb = feq_of(cub, w);
+    const float cu = cdot<qa>(ux, uy, uz);
+    const float three_cu = 3.0f * cu;
+    const float f45_cu2 = (4.5f * cu) * cu;
+    const float ea = w * (drho + r * ((f45_cu2 + three_cu) - f15_usq));
+    const float eb = w * (drho + r * ((f45_cu2 - three_cu) - f15_usq));
     const float fa = fv[qa], fb = fv[qb];
-    const float fp = half * (fa + fb);
-    const float fm = half * (fa - fb);
-    const float ep = half * (ea + eb);
-    const float em = half * (ea - eb);
-    const float rp = op * (fp - ep);
-    const float rm = om * (fm - em);
+    const float rp = hop * (halve(fa + fb) - halve(ea + eb));
+    const float rm = hom * (halve(fa - fb) - halve(ea - eb));
     float va = (fa - rp) - rm;
     float vb = (fb - rp) + rm;
     if (fon) {
-      const float sa = src_of(cua, cdot<qa>(Fc[0], Fc[1], Fc[2]), w);
-      const float sb = src_of(cub, cdot<qb>(Fc[0], Fc[1], Fc[2]), w);
-      const float sp = half * (sa + sb);
-      const float sm = half * (sa - sb);
-      const float cp_sp = cp * sp;
-      const float cm_sm = cm * sm;
+      const float cf = cdot<qa>(Fc[0], Fc[1], Fc[2]);
+      const float second = (9.0f * cu) * cf;
+      const float sa = w * (3.0f * (cf - uf) + second);
+      const float sb = w * (3.0f * (-cf - uf) + second);
+      const float cp_sp = hcp * halve(sa + sb);
+      const float cm_sm = hcm * halve(sa - sb);
       va = va + (cp_sp + cm_sm);
       vb = vb + (cp_sp - cm_sm);
     }
@@ -742,7 +731,7 @@ __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32
   if constexpr (KIND == 0) {
     float ux, uy, uz;
     moments<Q>(fv, Fm, fon, r, ux, uy, uz);
-    collide_trt<Q>(fv, r, ux, uy, uz, Fc, fon, op, cp, a.p);
+    collide_trt<Q, !Store<S>::kScaled>(fv, r, ux, uy, uz, Fc, fon, op, cp, a.p);
   } else if constexpr (Q == 19) {
     float ux, uy, uz;
     moments<Q>(fv, Fm, fon, r, ux, uy, uz);
@@ -832,18 +821,21 @@ __device__ __forceinline__ void hydro_tile(const HydroArgs& a) {
   if (t >= a.ntiles) return;
   const uint32_t te = __builtin_amdgcn_readfirstlane(a.tiles[t]);  // one tile per wave
   const uint32_t tile = te & kTileId;
-  if (!WRAP && a.lin) {
-    // linear tile: cells 64 tile .. 64 tile + 63 across row ends (no axis
-    // wraps, so every neighbour shift is the linear one)
+  if (a.lin) {
+    // linear tile: cells 64 tile .. 64 tile + 63 across row ends (where no
+    // axis wraps every neighbour shift is the linear one, elsewhere each lane
+    // takes its own coordinates)
     const uint32_t i = tile * 64 + (threadIdx.x & 63);
     if (i >= a.d.N || (te & ((threadIdx.x & 32) ? kTileDeadHi : kTileDeadLo))) return;
+    uint32_t x = 0u, y = 0u, z = 0u;
+    if constexpr (WRAP) cell_xyz(a.d, i, x, y, z);
     if (te & kTilePlain) {
-      cell_step<Q, S, KIND, ODD, FON, WRAP, true, true, WALE>(a, i, 0u, 0u, 0u, nullptr, 0u, a.p.F, a.p.F);
+      cell_step<Q, S, KIND, ODD, FON, WRAP, true, true, WALE>(a, i, x, y, z, nullptr, 0u, a.p.F, a.p.F);
     } else {
       const uint32_t c0 = tile * 64;
       const uint32_t lo = (te & kTileDeadLo) ? c0 + 32 : c0;
       const uint32_t hi = min((te & kTileDeadHi) ? c0 + 31 : c0 + 63, a.d.N - 1);
-      cell_step<Q, S, KIND, ODD, FON, WRAP, true, false, WALE>(a, i, 0u, 0u, 0u, a.mask + i, kMaskSolid | kMaskForced,
+      cell_step<Q, S, KIND, ODD, FON, WRAP, true, false, WALE>(a, i, x, y, z, a.mask + i, kMaskSolid | kMaskForced,
                                                          a.p.F, a.p.F, lo, hi, i);
     }
     return;
