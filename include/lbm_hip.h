@@ -435,7 +435,8 @@ int lbm_batch_torque_integral(lbm_batch* b, int reset, double* out);
  * and dJ/dnu per cell (nu = (1/omega_plus - 1/2)/3; omega_minus fixed, as
  * the omega field does).  Adjoint arithmetic is f64.  The fields end in the
  * state after the `steps` forward steps.  *forward_steps (nullable) counts
- * every forward step taken, the first pass included. */
+ * every forward step taken, the first pass included.  Gradients of domains of
+ * 2^29 cells and more are refused with LBM_ERR_UNSUPPORTED. */
 int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, double* J, double* dJ_domega,
                        double* dJ_dnu, int64_t* forward_steps);
 /* The checkpoint schedule used above, for inspection: `count` (action,

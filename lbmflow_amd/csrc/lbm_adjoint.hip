@@ -48,7 +48,8 @@ struct AdjArgs {
 // never stored: what lives through the kernel is lam* (19 f64) and f (19 fp32).
 // The form that held all three took 296 VGPRs, one wave per SIMD, and 240 us
 // on the 128^3 tank; this one 168, three waves, and 162 us (0.53 GB, 3.3 TB/s).
-// Solid cells are skipped: no fluid cell reads their adjoint, which stays zero.
+// Solid cells are skipped and their adjoint is left undefined: what a fluid
+// cell pulls from one is always replaced by its own reflected value.
 // FORCED cells (those of the force list) take the source's terms as well, in a
 // launch of their own over the list: in one kernel that rare branch sets the
 // register count.
@@ -67,8 +68,8 @@ __device__ __forceinline__ void adj_cell(const AdjArgs& a, uint32_t i, uint32_t 
     constexpr int q = decltype(qc)::value;
     f[q] = read_pop<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, ODD);
   });
-  // (plane bases are uniform, the per-lane part is one 32-bit byte offset: the
-  // f64 planes of a domain that fits the card stay below 4 GiB)
+  // (plane bases are uniform, the per-lane part is one 32-bit byte offset:
+  // lbm_adjoint_torque refuses domains whose f64 planes reach 4 GiB)
   const uint32_t at = i * 8u;
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;

@@ -2622,6 +2622,9 @@ int lbm_revolve_schedule(int steps, int snapshots, int* actions, int capacity, i
 int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, double* J, double* dJ_domega,
                        double* dJ_dnu, int64_t* forward_steps) {
   if (!fl || steps < 1 || window < 1 || window > steps || snapshots < 0 || !J) return LBM_ERR_INVALID;
+  // the reverse kernel's lane offsets into an f64 plane are 32-bit byte offsets
+  if ((dJ_domega || dJ_dnu) && fl->d.N >= (1u << 29))
+    return fail(fl->ctx, LBM_ERR_UNSUPPORTED, "the adjoint takes domains below 2^29 cells (%u given)", fl->d.N);
   if (!fl->ibm) return fail(fl->ctx, LBM_ERR_STATE, "the torque adjoint needs a rotating body");
   if (fl->Q != 19 || fl->collision == LBM_COLLISION_CM)
     return fail(fl->ctx, LBM_ERR_UNSUPPORTED, "the adjoint is implemented for D3Q19 TRT/BGK");

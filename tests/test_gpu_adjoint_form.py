@@ -58,3 +58,17 @@ def test_directional_gradient_matches_differences(collision, periodic, dims):
     ad = float(np.dot(a["dJ_dnu"], d))
     # fp32 forward: J carries about 1e-7 of rounding against steps of 1e-2
     assert abs(ad - fd) <= 2e-3 * abs(fd) + 1e-5 * abs(a["J"])
+
+
+def test_domain_beyond_the_lane_offset_is_refused():
+    """An f64 plane of 2^29 cells is 4 GiB, past the reverse kernel's 32-bit
+    byte offset: the gradient is refused before anything else is looked at (no
+    body is registered here), the forward-only call as before."""
+    s = L.Solver(19, (1024, 1024, 512), nu=0.02, storage="f16", periodic=(True,) * 3)
+    with pytest.raises(L.LbmError) as e:
+        s.adjoint_torque(2, 1, 1)
+    assert e.value.code == -2 and "2^29" in str(e.value)
+    with pytest.raises(L.LbmError) as e:
+        s.adjoint_torque(2, 1, 1, gradients=False)
+    assert e.value.code == -5  # no body
+    s.close()
