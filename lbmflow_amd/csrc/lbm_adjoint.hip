@@ -18,6 +18,8 @@
 // omega_bar), of F_cur (Fbar) and of F_mom (Gout) at forced cells.  All
 // adjoint arithmetic is f64; the forward state is the stored fp32 (or
 // 16-bit) populations, read in the parity-dependent AA layout.
+#include <algorithm>
+
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
 
@@ -287,13 +289,16 @@ hipError_t launch_nu_bar(uint32_t n, const double* omega_bar, const float* omega
 }
 
 __global__ void k_fill_d(double* p, size_t n, double v) {
-  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) p[k] = v;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) p[k] = v;
 }
 
 hipError_t launch_fill_f64(double* p, size_t n, double v, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_d, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
+  // one work-item per double would pass the 2^32 work-items a launch may have
+  // from 148 M cells on (29 doubles per cell are zeroed at once)
+  const size_t blocks = std::min<size_t>((n + 255) / 256, 65536);
+  hipLaunchKernelGGL(k_fill_d, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
   return hipGetLastError();
 }
 

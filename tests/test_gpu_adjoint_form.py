@@ -72,3 +72,25 @@ def test_domain_beyond_the_lane_offset_is_refused():
         s.adjoint_torque(2, 1, 1, gradients=False)
     assert e.value.code == -5  # no body
     s.close()
+
+
+def test_large_domain_gives_the_small_domain_gradient():
+    """148.6 M cells: the zeroed adjoint arrays hold more than 2^32 doubles.
+    What the body of a resting fluid reaches in four steps is the same cells in
+    a small domain, so the gradient there has the same bits and is zero
+    elsewhere."""
+    rng = np.random.RandomState(4)
+    c = np.array([32.0, 32.0, 24.0])
+    pos = c + rng.uniform(-3.0, 3.0, (20, 3))
+    out = []
+    for nz in (48, 36272):
+        s = L.Solver(19, (64, 64, nz), nu=0.05, storage="f16", periodic=(True,) * 3)
+        s.set_rotating_body(pos, 0.3 * np.ones(20), c, (0.0, 0.0, 0.012))
+        out.append(s.adjoint_torque(4, 2, 1))
+        s.close()
+    small, large = out
+    n = small["dJ_dnu"].size
+    assert 29 * large["dJ_dnu"].size > 2 ** 32
+    assert small["J"] == large["J"] != 0.0 and small["dJ_domega"] == large["dJ_domega"] != 0.0
+    assert np.any(small["dJ_dnu"] != 0.0)
+    assert np.array_equal(large["dJ_dnu"][:n], small["dJ_dnu"]) and not np.any(large["dJ_dnu"][n:])
