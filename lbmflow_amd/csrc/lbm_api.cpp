@@ -1269,12 +1269,6 @@ static int check_steppable(lbm_fields* fl) {
                 fl->uncovered);
   if (fl->open_face_cells && !fl->scalars.empty())
     return fail(fl->ctx, LBM_ERR_UNSUPPORTED, "scalar distributions do not take open faces on this path");
-  // the closure inside the step writes fluid cells: the others hold the
-  // laminar rate, as the closure's own pass gives it
-  if (fl->wale_fill && wale_in_step(fl)) {
-    HIPCHK(fl->ctx, launch_fill_f32(fl->omega, fl->d.N, 1.0f / (3.0f * (float)wale_nu(fl) + 0.5f), fl->ctx->stream));
-    fl->wale_fill = false;
-  }
   if (!fl->probe_host.empty() && !fl->probe_built) return probe_build(fl);
   return LBM_OK;
 }
@@ -1433,6 +1427,16 @@ static int open_faces_step(lbm_fields* fl) {
   return LBM_OK;
 }
 
+// Before a span's first step: the closure inside the step writes fluid cells
+// only, so the solid ones get the laminar rate here, as the closure's own pass
+// gives it.
+static int wale_solid_rate(lbm_fields* fl) {
+  if (!fl->wale_fill || !wale_in_step(fl)) return LBM_OK;
+  HIPCHK(fl->ctx, launch_wale_solid(fl->d.N, fl->mask, (float)wale_nu(fl), fl->omega, fl->ctx->stream));
+  fl->wale_fill = false;
+  return LBM_OK;
+}
+
 // Whether a step may leave its scalar step to the next step's velocity pass:
 // a single D3Q7 scalar beside the closure inside the step.
 static bool scalar_rides(const lbm_fields* fl) {
@@ -1528,6 +1532,7 @@ static int finish_scalars(lbm_fields* fl) {
 int lbm_run_span(lbm_fields* fl, int steps) {
   if (!fl || steps < 0) return LBM_ERR_INVALID;
   int rc = check_steppable(fl);
+  if (!rc && steps > 0) rc = wale_solid_rate(fl);
   if (rc) return rc;
   for (int k = 0; k < steps; ++k) {
     rc = hydro_step(fl);
@@ -1556,6 +1561,8 @@ int lbm_run_ibm_span(lbm_fields* fl, int steps, int use_graph, double* torque, l
   int rc = check_steppable(fl);
   if (rc) return rc;
   if (steps == 0) return LBM_OK;
+  rc = wale_solid_rate(fl);
+  if (rc) return rc;
   if (fl->field_present && fl->field_uniform) {  // the clear must refresh the cached moments
     rc = lbm_clear_force_field(fl);
     if (rc) return rc;

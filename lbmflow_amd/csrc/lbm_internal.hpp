@@ -251,6 +251,8 @@ struct ScalarStepArgs;
 hipError_t launch_wale_local(int Q, int storage, const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s);
 hipError_t launch_wale_omega(const WaleFields& a, float cw_delta_sq, float nu0, float nut_max, float* omega,
                              float* nut, uint32_t* stats, hipStream_t s);
+// the laminar rate into the omega field's solid cells
+hipError_t launch_wale_solid(uint32_t n, const uint32_t* mask, float nu0, float* omega, hipStream_t s);
 // One passive-scalar step of a domain (lbm_scalar.hpp).
 struct ScalarStepArgs {
   const float* h;   // Qs planes: this step's distribution

@@ -290,6 +290,17 @@ hipError_t launch_wale_local(int Q, int storage, const WaleFields& a, const Scal
   return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void k_wale_solid(uint32_t n, const uint32_t* mask, float nu0, float* omega) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && (mask[i] & kMaskSolid)) omega[i] = wale_omega(nu0, 0.0f);
+}
+
+hipError_t launch_wale_solid(uint32_t n, const uint32_t* mask, float nu0, float* omega, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_wale_solid, dim3((n + 255) / 256), dim3(256), 0, s, n, mask, nu0, omega);
+  return hipGetLastError();
+}
+
 __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) p[k] = 0u;

@@ -90,6 +90,34 @@ def test_tiles_autotuned_under_the_closure_leave_the_field():
     s.close()
 
 
+def test_calls_without_a_step_leave_the_field():
+    """After the closure is switched on (again) the installed field stands until
+    a step writes it: spans of no step and the autotuner leave it alone."""
+    tc = cases.tank_case(28, nu=0.004)
+    s = L.Solver(27, (28,) * 3, nu=0.004, collision="cm", solid=tc["solid"])
+    s.set_rotating_body(tc["pos"], tc["w"], tc["c"], (0.0, 0.0, tc["omega"]))
+    s.set_wale(True)
+    s.run_with_ibm(3)
+    computed = s.omega_field()
+    given = (1.0 + 0.2 * np.random.RandomState(1).rand(s.n)).astype(np.float32)
+    for field in (computed, given):
+        s.set_omega_field(field)
+        s.set_wale(True)
+        for call in (lambda: s.run(0), lambda: s.run_with_ibm(0), lambda: s.autotune_tiles(4)):
+            call()
+            assert np.array_equal(s.omega_field(), field)
+    s.set_wale(False)
+    assert np.array_equal(s.omega_field(), given)
+    # and a step writes all of it, the solid cells included
+    s.set_wale(True)
+    s.run_with_ibm(1)
+    solid = tc["solid"].reshape(-1) != 0
+    rate = np.float32(1.0) / (np.float32(3.0) * np.float32(0.004) + np.float32(0.5))
+    assert np.abs(s.omega_field()[solid] - rate).max() <= 2.0 ** -21  # last bits of the sum (2^-24) and of a quotient near 2
+    assert not np.array_equal(s.omega_field()[~solid], given[~solid])
+    s.close()
+
+
 @pytest.mark.parametrize("Q,collision", [(27, "cm"), (19, "trt")])
 def test_tank_with_body_follows_the_oracle(Q, collision):
     tc = cases.tank_case(30, collision=collision, Q=Q, nu=0.004)
