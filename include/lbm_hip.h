@@ -138,7 +138,8 @@ int lbm_access_copy(lbm_ctx* ctx, int width, int offset_elems, size_t bytes, int
 int lbm_fields_alloc(lbm_ctx* ctx, int Q, int storage, const int dims[3], const int periodic[3],
                      lbm_fields** out);
 void lbm_fields_free(lbm_fields* fl);
-/* Device bytes held by this domain. */
+/* Device bytes held by this domain.  Not counted: the context's read-back
+ * workspace (at most 64 MiB, as much as its largest read needed). */
 size_t lbm_fields_device_bytes(const lbm_fields* fl);
 
 /* Solver::build mask distribution, solver.rs:1829-1848: solid (1 byte per

@@ -535,6 +535,17 @@ int read_array(lbm_fields* fl, void* dst, const void* src, size_t bytes) {
   return LBM_OK;
 }
 
+// planes of the domain's cells, produced in pieces, to caller memory
+int read_planes(lbm_fields* fl, uint32_t planes, const std::function<float*(uint32_t)>& out,
+                const std::function<hipError_t(uint32_t, uint32_t, float*)>& produce) {
+  const hipError_t read_back =
+      fl->ctx->rb.read_planes(fl->ctx->device, fl->ctx->stream, fl->d.N, planes, out, produce);
+  if (read_back == hipErrorOutOfMemory)
+    return fail(fl->ctx, LBM_ERR_NOMEM, "no device memory for a read-back workspace");
+  HIPCHK(fl->ctx, read_back);
+  return LBM_OK;
+}
+
 // Cached moments now carry the current field (Backend::update_moments).
 int refresh_moments(lbm_fields* fl) {
   if (fl->F_mom && !fl->flist_host.empty())
@@ -887,22 +898,12 @@ int lbm_stage_in(lbm_fields* fl, const float* f) {
 
 int lbm_stage_out(lbm_fields* fl, float* f) {
   if (!fl || !f) return LBM_ERR_INVALID;
-  hipStream_t s = fl->ctx->stream;
-  Readback& rb = fl->ctx->rb;
-  float* w = (float*)rb.work();
-  if (!w) return fail(fl->ctx, LBM_ERR_NOMEM, "read-back workspace of %zu bytes", Readback::kWorkBytes);
-  // pieces of as many cells as the workspace holds Q planes of
-  const uint32_t N = fl->d.N, Q = (uint32_t)fl->Q;
-  const uint32_t per = (uint32_t)(Readback::kWorkBytes / 4 / Q) / 1024 * 1024;
-  const int pieces = (int)((N + per - 1) / per);
-  const hipError_t read_back = rb.read(fl->ctx->device, s, pieces, [&](int p, std::vector<Readback::Seg>& segs) {
-    const uint32_t i0 = (uint32_t)p * per, cnt = std::min(per, N - i0);
-    for (uint32_t q = 0; q < Q; ++q)
-      segs.push_back({f + (size_t)q * N + i0, w + (size_t)q * cnt, (size_t)cnt * 4});
-    return launch_stage(fl->Q, fl->storage, 1, fl->parity, fl->d, fl->f, w, fl->mask, i0, cnt, s);
-  });
-  HIPCHK(fl->ctx, read_back);
-  return LBM_OK;
+  const uint32_t N = fl->d.N;
+  return read_planes(
+      fl, (uint32_t)fl->Q, [&](uint32_t q) { return f + (size_t)q * N; },
+      [&](uint32_t i0, uint32_t cnt, float* w) {
+        return launch_stage(fl->Q, fl->storage, 1, fl->parity, fl->d, fl->f, w, fl->mask, i0, cnt, fl->ctx->stream);
+      });
 }
 
 int lbm_init_with(lbm_fields* fl, const float* rho, const float* u) {
@@ -1691,22 +1692,13 @@ int64_t lbm_time(const lbm_fields* fl) { return fl ? fl->time : -1; }
 
 int lbm_read_moments(lbm_fields* fl, float* rho, float* ux, float* uy, float* uz) {
   if (!fl || !rho || !ux || !uy || !uz) return LBM_ERR_INVALID;
-  hipStream_t s = fl->ctx->stream;
-  Readback& rb = fl->ctx->rb;
-  float* w = (float*)rb.work();
-  if (!w) return fail(fl->ctx, LBM_ERR_NOMEM, "read-back workspace of %zu bytes", Readback::kWorkBytes);
-  const uint32_t N = fl->d.N;
-  const uint32_t per = (uint32_t)(Readback::kWorkBytes / 16);
-  const int pieces = (int)((N + per - 1) / per);
   float* const out[4] = {rho, ux, uy, uz};
-  const hipError_t read_back = rb.read(fl->ctx->device, s, pieces, [&](int p, std::vector<Readback::Seg>& segs) {
-    const uint32_t i0 = (uint32_t)p * per, cnt = std::min(per, N - i0);
-    for (int k = 0; k < 4; ++k) segs.push_back({out[k] + i0, w + (size_t)k * cnt, (size_t)cnt * 4});
-    return launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, i0, cnt, w,
-                          w + cnt, w + 2 * (size_t)cnt, w + 3 * (size_t)cnt, s);
-  });
-  HIPCHK(fl->ctx, read_back);
-  return LBM_OK;
+  return read_planes(
+      fl, 4, [&](uint32_t k) { return out[k]; },
+      [&](uint32_t i0, uint32_t cnt, float* w) {
+        return launch_moments(fl->Q, fl->storage, fl->parity, fl->d, fl->f, fl->mask, fl->F_mom, fl->hp, i0, cnt, w,
+                              w + cnt, w + 2 * (size_t)cnt, w + 3 * (size_t)cnt, fl->ctx->stream);
+      });
 }
 
 int lbm_read_moments_noalloc(lbm_fields* fl, float* rho, float* ux, float* uy, float* uz) {

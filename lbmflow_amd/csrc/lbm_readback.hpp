@@ -10,8 +10,9 @@
 //
 // One object per context; calls on a context are serialized by the caller,
 // different contexts share nothing.  The pinned slots and the workspace are
-// allocated at first use, bounded (kSlots * kSlotBytes, kWorkBytes) and given
-// back with the context.  Threads live only inside a call.
+// allocated at first use, as large as the largest read so far needs and at most
+// kSlots * kSlotBytes and kWorkBytes, and given back with the context.  Threads
+// live only inside a call.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -19,6 +20,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
+#include <cstdint>
 #include <cstring>
 #include <functional>
 #include <mutex>
@@ -37,6 +39,7 @@ class Readback {
   static constexpr size_t kSlotBytes = (size_t)2 << 20;
   static constexpr int kSlots = 24;
   static constexpr size_t kWorkBytes = (size_t)64 << 20;
+  static constexpr size_t kMinWorkBytes = (size_t)64 << 10;
   static constexpr int kThreads = 12;  // of the 16 host cores a GPU comes with
 
   Readback() = default;
@@ -48,10 +51,24 @@ class Readback {
     if (work_) (void)hipFree(work_);
   }
 
-  // Device workspace of kWorkBytes for the pieces; null when it cannot be had.
-  void* work() {
-    if (!work_ && hipMalloc(&work_, kWorkBytes) != hipSuccess) work_ = nullptr;
-    return work_;
+  // `planes` planes of n floats to out(plane).  produce(i0, cnt, w) enqueues on
+  // `s` what writes the values i0 .. i0 + cnt - 1 of each plane to w + plane *
+  // cnt.  hipErrorOutOfMemory: no workspace could be had.
+  hipError_t read_planes(int device, hipStream_t s, uint32_t n, uint32_t planes,
+                         const std::function<float*(uint32_t)>& out,
+                         const std::function<hipError_t(uint32_t, uint32_t, float*)>& produce) {
+    size_t have = 0;
+    float* w = (float*)work((size_t)planes * n * sizeof(float), &have);
+    if (!w) return hipErrorOutOfMemory;
+    size_t per = have / sizeof(float) / planes;
+    per = per < n ? per / 64 * 64 : n;
+    const int pieces = (int)((n + per - 1) / per);
+    return read(device, s, pieces, [&](int p, std::vector<Seg>& segs) {
+      const uint32_t i0 = (uint32_t)(p * per), cnt = (uint32_t)std::min<size_t>(per, n - i0);
+      for (uint32_t k = 0; k < planes; ++k)
+        segs.push_back({out(k) + i0, w + (size_t)k * cnt, (size_t)cnt * sizeof(float)});
+      return produce(i0, cnt, w);
+    });
   }
 
   // Runs produce(p, segs) for p = 0 .. pieces - 1 in order.  Each call enqueues
@@ -63,16 +80,7 @@ class Readback {
     std::vector<Seg> segs;
     segs.reserve(64);  // nothing is allocated while threads run
     hipError_t e = hipSuccess;
-    if (!ensure_slots()) {  // no pinned memory: the runtime's own copies
-      for (int p = 0; p < pieces && e == hipSuccess; ++p) {
-        segs.clear();
-        e = produce(p, segs);
-        for (const Seg& g : segs)
-          if (e == hipSuccess) e = hipMemcpyAsync(g.dst, g.src, g.bytes, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-      }
-      return e;
-    }
+    bool slots = false;
     Job job;
     std::vector<std::thread> pool;
     pool.reserve(kThreads);
@@ -82,7 +90,16 @@ class Readback {
       if (e != hipSuccess) break;
       size_t total = 0;
       for (const Seg& g : segs) total += g.bytes;
-      if (pieces == 1 && total <= kSlotBytes) {  // one slot, one wait, no thread
+      const bool one = pieces == 1 && total <= kSlotBytes;
+      if (p == 0) slots = ensure_slots(one ? 1 : kSlots);
+      if (!slots) {  // no pinned memory: the runtime's own copies
+        for (const Seg& g : segs)
+          if (e == hipSuccess) e = hipMemcpyAsync(g.dst, g.src, g.bytes, hipMemcpyDeviceToHost, s);
+        const hipError_t w = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = w;
+        continue;
+      }
+      if (one) {  // one slot, one wait, no thread
         size_t at = 0;
         for (const Seg& g : segs) {
           if (e == hipSuccess) e = hipMemcpyAsync(pin_ + at, g.src, g.bytes, hipMemcpyDeviceToHost, s);
@@ -206,35 +223,55 @@ class Readback {
     }
   }
 
-  bool ensure_slots() {
-    if (pin_) return true;
-    if (failed_) return false;
+  // At least n slots (1: a small read; kSlots: any other).  Asked for again
+  // only where fewer had been refused.
+  bool ensure_slots(int n) {
+    if (slots_ >= n) return true;
+    if (refused_ && n >= refused_) return false;
     void* p = nullptr;
-    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocDefault) != hipSuccess) {
+    bool ok = hipHostMalloc(&p, kSlotBytes * n, hipHostMallocDefault) == hipSuccess;
+    while (ok && n > 1 && (int)ev_.size() < n) {
+      hipEvent_t e;
+      ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+      if (ok) ev_.push_back(e);
+    }
+    if (!ok) {
       (void)hipGetLastError();
-      failed_ = true;
+      if (p) (void)hipHostFree(p);
+      refused_ = n;
       return false;
     }
-    for (int k = 0; k < kSlots; ++k) {
-      hipEvent_t e;
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        for (hipEvent_t x : ev_) (void)hipEventDestroy(x);
-        ev_.clear();
-        (void)hipHostFree(p);
-        failed_ = true;
-        return false;
-      }
-      ev_.push_back(e);
-    }
+    if (pin_) (void)hipHostFree(pin_);
     pin_ = (char*)p;
+    slots_ = n;
     return true;
   }
 
+  // Device workspace: as much as asked for up to kWorkBytes, or what a full
+  // card still has of it; null when not even kMinWorkBytes can be had.
+  void* work(size_t want, size_t* have) {
+    want = std::min(std::max(want, kMinWorkBytes), kWorkBytes);
+    if (work_bytes_ < want) {
+      if (work_) (void)hipFree(work_);
+      for (work_ = nullptr, work_bytes_ = want; hipMalloc(&work_, work_bytes_) != hipSuccess;) {
+        (void)hipGetLastError();
+        work_ = nullptr;
+        if (work_bytes_ <= kMinWorkBytes) {
+          work_bytes_ = 0;
+          break;
+        }
+        work_bytes_ = std::max(work_bytes_ / 2, kMinWorkBytes);
+      }
+    }
+    *have = work_bytes_;
+    return work_;
+  }
+
   char* pin_ = nullptr;
+  int slots_ = 0, refused_ = 0;
   std::vector<hipEvent_t> ev_;
   void* work_ = nullptr;
-  bool failed_ = false;
+  size_t work_bytes_ = 0;
 };
 
 }  // namespace lbm

@@ -39,3 +39,25 @@ def test_moments_and_populations_in_pieces(Q, dims):
         # each of at most Q roundings is below 2^-24 of the partial sums' bound Q * 5e-3
         assert np.abs(u - ref).max() <= 2.0 * Q * 2.0 ** -24 * Q * 5e-3
     s.close()
+
+
+def test_small_domain_holds_little_device_memory():
+    """Reads of a 16^3 domain keep what they need, not the workspace's bound."""
+    import ctypes as C
+
+    import lbmflow_amd as L
+
+    ctx = L.Context(0)
+
+    def free_bytes():  # by the runtime the library is linked with
+        f, t = C.c_size_t(), C.c_size_t()
+        assert ctx.lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    s = L.Solver(19, (16, 16, 16), nu=0.05, periodic=(True,) * 3, ctx=ctx)
+    s.run(2)
+    before = free_bytes()
+    s.moments()
+    s.populations()
+    assert before - free_bytes() <= 8 << 20
+    s.close()
