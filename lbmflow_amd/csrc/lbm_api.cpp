@@ -129,6 +129,8 @@ struct lbm_fields {
   // the last step's scalar step is left to the next step's velocity pass
   // (inside a span only)
   bool scalar_pending = false;
+  // steps leave the scalars alone (steps taken again by the adjoint)
+  bool scalars_held = false;
   size_t bytes = 0;
 };
 
@@ -1504,6 +1506,7 @@ static int hydro_step(lbm_fields* fl) {
   }
   fl->parity ^= 1;
   fl->time += 1;
+  if (fl->scalars_held) return LBM_OK;
   if (scalar_rides(fl)) {
     fl->scalar_pending = true;
     return LBM_OK;
@@ -2669,6 +2672,7 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
   auto cleanup = [&]() {
     const std::string err = fl->ctx->err;  // the failure being reported
     if (reversing) (void)snap_restore(fl, fin);
+    fl->scalars_held = false;
     (void)hipStreamSynchronize(s);
     fl->ctx->err = err;
     if (slab) (void)hipFree(slab);
@@ -2728,8 +2732,10 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     return LBM_OK;
   }
   ADJ_TRY(snap_save(fl, fin));
-  // reverse pass
+  // reverse pass: the snapshots hold the flow alone, so the steps taken again
+  // leave the scalars as the forward pass left them
   reversing = true;
+  fl->scalars_held = true;
   int64_t advanced = steps;
   const double tq_bar = 1.0 / window;
   // the snapshot slot the device state still equals (the schedule restores
@@ -2773,7 +2779,6 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
   if (dJ_domega) *dJ_domega = ob;
   if (forward_steps) *forward_steps = advanced;
   ADJ_TRY(snap_restore(fl, fin));
-  ADJ_TRY(finish_scalars(fl));
   ADJ_HIP(hipStreamSynchronize(s));
   reversing = false;
   cleanup();

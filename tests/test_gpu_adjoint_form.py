@@ -94,3 +94,33 @@ def test_large_domain_gives_the_small_domain_gradient():
     assert small["J"] == large["J"] != 0.0 and small["dJ_domega"] == large["dJ_domega"] != 0.0
     assert np.any(small["dJ_dnu"] != 0.0)
     assert np.array_equal(large["dJ_dnu"][:n], small["dJ_dnu"]) and not np.any(large["dJ_dnu"][n:])
+
+
+@pytest.mark.parametrize("snapshots", [0, 3])
+def test_gradient_leaves_the_tracers_of_the_forward_steps(snapshots):
+    """The steps that the reverse pass takes again do not move the passive
+    scalars: the concentrations after the call are those after the same steps
+    without it, bit for bit, and so are those of the steps that follow."""
+    n, steps = 24, 9
+    tc = cases.tank_case(n, nu=0.02, collision="trt", Q=19)
+
+    def solver():
+        s = L.Solver(19, (n,) * 3, nu=0.02, collision="trt", solid=tc["solid"])
+        s.set_rotating_body(tc["pos"], tc["w"], tc["c"], (0.0, 0.0, tc["omega"]))
+        for lat in ("d3q7", "hydro"):
+            s.set_scalar_concentration(s.enable_scalar_distribution(0.01, lat), tc["blob"])
+        return s
+
+    a, b = solver(), solver()
+    res = a.adjoint_torque(steps, 4, snapshots)
+    assert res["forward_steps"] > steps
+    b.run_with_ibm(steps)
+    for k in (0, 1):
+        assert np.array_equal(a.gather_scalar_concentration(k), b.gather_scalar_concentration(k))
+    for s in (a, b):
+        s.run_with_ibm(3)
+    for k in (0, 1):
+        assert np.array_equal(a.gather_scalar_concentration(k), b.gather_scalar_concentration(k))
+    assert a.time == b.time
+    a.close()
+    b.close()
