@@ -129,8 +129,8 @@ struct lbm_fields {
   // the last step's scalar step is left to the next step's velocity pass
   // (inside a span only)
   bool scalar_pending = false;
-  // steps leave the scalars alone (steps taken again by the adjoint)
-  bool scalars_held = false;
+  // steps taken again by the adjoint: they leave the scalars and the probe alone
+  bool replay = false;
   size_t bytes = 0;
 };
 
@@ -1467,7 +1467,8 @@ static int hydro_step(lbm_fields* fl) {
     int rc = wale_enqueue(fl, fl->wale_cw2, fl->wale_nut_max, nullptr, nullptr);
     if (rc) return rc;
   }
-  if (fl->probe_built) {
+  const bool probe = fl->probe_built && !fl->replay;
+  if (probe) {
     int rc = probe_launch(fl, 0);
     if (rc) return rc;
   }
@@ -1488,7 +1489,7 @@ static int hydro_step(lbm_fields* fl) {
     fl->ev_used += 2;
   }
   if (a.nlist) HIPCHK(fl->ctx, launch_hydro_list(fl->Q, fl->storage, fl->collision, fl->parity, a, s));
-  if (fl->probe_built) {  // before the open faces, as the stream accumulates it
+  if (probe) {  // before the open faces, as the stream accumulates it
     int rc = probe_launch(fl, 1);
     if (rc) return rc;
   }
@@ -1506,7 +1507,7 @@ static int hydro_step(lbm_fields* fl) {
   }
   fl->parity ^= 1;
   fl->time += 1;
-  if (fl->scalars_held) return LBM_OK;
+  if (fl->replay) return LBM_OK;
   if (scalar_rides(fl)) {
     fl->scalar_pending = true;
     return LBM_OK;
@@ -2665,14 +2666,22 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
   Snapshot fin;
   double *lamA = nullptr, *lamB = nullptr, *obar = nullptr, *Fbar = nullptr, *G0 = nullptr, *G1 = nullptr,
          *wbar = nullptr;
+  float* fin_F = nullptr;       // force field at the listed cells,
+  double* fin_integ = nullptr;  // torque integral after the forward pass
   char* slab = nullptr;
   // a failure after the forward pass puts the final state back (best
   // effort) before the allocation is freed
   bool reversing = false;
+  auto restore_final = [&]() -> int {
+    int r = snap_restore(fl, fin);
+    if (r) return r;
+    HIPCHK(fl->ctx, launch_list_pack(fl->flist, (uint32_t)fl->flist_host.size(), fl->F_cur, fin_F, 1, s));
+    return ibm_integral_copy(view_of(fl), fl->ibm, fin_integ, 1);
+  };
   auto cleanup = [&]() {
     const std::string err = fl->ctx->err;  // the failure being reported
-    if (reversing) (void)snap_restore(fl, fin);
-    fl->scalars_held = false;
+    if (reversing) (void)restore_final();
+    fl->replay = false;
     (void)hipStreamSynchronize(s);
     fl->ctx->err = err;
     if (slab) (void)hipFree(slab);
@@ -2694,7 +2703,7 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     const size_t fb = up(fl->f_bytes), lb = up(3 * sizeof(float) * std::max<size_t>(1, fl->flist_host.size()));
     // zeroed: lamA, the force adjoints, omega_bar, the rotation rate's
     const size_t nz = Q * N + 9 * N + N + 1;
-    const size_t bytes = (slots + 1) * (fb + lb) + up(nz * sizeof(double)) + Q * N * sizeof(double);
+    const size_t bytes = (slots + 1) * (fb + lb) + lb + 256 + up(nz * sizeof(double)) + Q * N * sizeof(double);
     if (hipMalloc((void**)&slab, bytes) != hipSuccess) {
       slab = nullptr;
       return fail(fl->ctx, LBM_ERR_NOMEM, "adjoint workspace of %zu bytes (%zu snapshots)", bytes, slots + 1);
@@ -2711,6 +2720,8 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     }
     fin.f = take(fb);
     fin.F_mom = (float*)take(lb);
+    fin_F = (float*)take(lb);
+    fin_integ = (double*)take(256);  // one body
     lamA = (double*)take(up(nz * sizeof(double)));
     lamB = (double*)take(Q * N * sizeof(double));
     G0 = lamA + Q * N;
@@ -2732,10 +2743,13 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     return LBM_OK;
   }
   ADJ_TRY(snap_save(fl, fin));
-  // reverse pass: the snapshots hold the flow alone, so the steps taken again
-  // leave the scalars as the forward pass left them
+  ADJ_HIP(launch_list_pack(fl->flist, (uint32_t)fl->flist_host.size(), fl->F_cur, fin_F, 0, s));
+  ADJ_TRY(ibm_integral_copy(view_of(fl), fl->ibm, fin_integ, 0));
+  // reverse pass: the steps taken again leave the scalars and the probed force
+  // as the forward pass left them; the body's force and torque integral, which
+  // they advance, are put back with the flow
   reversing = true;
-  fl->scalars_held = true;
+  fl->replay = true;
   int64_t advanced = steps;
   const double tq_bar = 1.0 / window;
   // the snapshot slot the device state still equals (the schedule restores
@@ -2778,7 +2792,7 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
   ADJ_HIP(hipStreamSynchronize(s));
   if (dJ_domega) *dJ_domega = ob;
   if (forward_steps) *forward_steps = advanced;
-  ADJ_TRY(snap_restore(fl, fin));
+  ADJ_TRY(restore_final());
   ADJ_HIP(hipStreamSynchronize(s));
   reversing = false;
   cleanup();

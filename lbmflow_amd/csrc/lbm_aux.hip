@@ -1506,6 +1506,12 @@ int ibm_torque_integral(const FieldsView& v, IbmState* s, int reset, double* out
   return LBM_OK;
 }
 
+int ibm_integral_copy(const FieldsView& v, IbmState* s, double* buf, int dir) {
+  AUXCHK(v, hipMemcpyAsync(dir ? s->integ : buf, dir ? buf : s->integ, 4 * (size_t)s->K * sizeof(double),
+                           hipMemcpyDeviceToDevice, v.stream));
+  return LBM_OK;
+}
+
 size_t ibm_ring_entry_bytes() { return sizeof(IbmDevDiag); }
 
 int ibm_ring_read(const FieldsView& v, const void* ring, uint32_t n, lbm_ibm_diag* out) {

@@ -79,6 +79,8 @@ size_t ibm_ring_entry_bytes();
 // Running f64 torque integral per instance: out[4k + c] = sum of torque c
 // over the updates since the last reset, out[4k + 3] = their count.
 int ibm_torque_integral(const FieldsView& v, IbmState* s, int reset, double* out);
+// the integrals (4 doubles per instance) to a device buffer (dir 0) or back (dir 1)
+int ibm_integral_copy(const FieldsView& v, IbmState* s, double* buf, int dir);
 // Adjoint support (single body).  ibm_enqueue_recorded is ibm_enqueue that
 // also keeps every sweep's impulses and du for ibm_adjoint, which runs the
 // sweeps backwards: Fbar (+ Gbar, nullable) is the adjoint of the force

@@ -124,3 +124,34 @@ def test_gradient_leaves_the_tracers_of_the_forward_steps(snapshots):
     assert a.time == b.time
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("snapshots", [0, 3])
+def test_gradient_leaves_the_state_of_the_forward_steps(snapshots):
+    """Populations, force field, torque integral and probed force after the
+    call are those after the same steps without it, bit for bit, also for a
+    plain step that still uses the force field."""
+    n, steps = 24, 9
+    tc = cases.tank_case(n, nu=0.02, collision="trt", Q=19)
+
+    def solver():
+        s = L.Solver(19, (n,) * 3, nu=0.02, collision="trt", solid=tc["solid"])
+        s.set_rotating_body(tc["pos"], tc["w"], tc["c"], (0.0, 0.0, tc["omega"]))
+        s.set_force_probe(tc["solid"])
+        return s
+
+    def state(s):
+        torque, updates = s.torque_integral()
+        return [s.populations(), s.body_force_field(), torque, s.probed_force(), np.array([updates, s.time])]
+
+    a, b = solver(), solver()
+    assert a.adjoint_torque(steps, 4, snapshots)["forward_steps"] > steps
+    b.run_with_ibm(steps)
+    for call in (None, lambda s: s.run(1), lambda s: s.run_with_ibm(2)):
+        for s in (a, b):
+            if call:
+                call(s)
+        for x, y in zip(state(a), state(b)):
+            assert np.array_equal(x, y)
+    a.close()
+    b.close()
