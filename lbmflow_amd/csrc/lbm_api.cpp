@@ -194,7 +194,7 @@ int fail(lbm_ctx* c, int code, const char* fmt, ...) {
 
 int dev_alloc(lbm_fields* fl, void** p, size_t bytes) {
   if (bytes == 0) bytes = 1;
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = gpu_malloc(p, bytes, &fl->ctx->rb);
   if (e != hipSuccess) {
     *p = nullptr;
     return fail(fl->ctx, LBM_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
@@ -618,8 +618,8 @@ int lbm_stream_copy(lbm_ctx* ctx, size_t bytes, int iterations, double* gbps) {
   if (!ctx || !gbps || iterations <= 0 || bytes < 16) return LBM_ERR_INVALID;
   bytes &= ~(size_t)15;
   void *a = nullptr, *b = nullptr;
-  if (hipMalloc(&a, bytes) != hipSuccess) return fail(ctx, LBM_ERR_NOMEM, "stream copy: hipMalloc failed");
-  if (hipMalloc(&b, bytes) != hipSuccess) {
+  if (gpu_malloc(&a, bytes, &ctx->rb) != hipSuccess) return fail(ctx, LBM_ERR_NOMEM, "stream copy: hipMalloc failed");
+  if (gpu_malloc(&b, bytes, &ctx->rb) != hipSuccess) {
     (void)hipFree(a);
     return fail(ctx, LBM_ERR_NOMEM, "stream copy: hipMalloc failed");
   }
@@ -652,8 +652,8 @@ int lbm_access_copy(lbm_ctx* ctx, int width, int offset_elems, size_t bytes, int
   const size_t n = bytes / (size_t)width;
   const size_t alloc = n * (size_t)width + 256;  // room for the offset element
   void *a = nullptr, *b = nullptr;
-  if (hipMalloc(&a, alloc) != hipSuccess) return fail(ctx, LBM_ERR_NOMEM, "access copy: hipMalloc failed");
-  if (hipMalloc(&b, alloc) != hipSuccess) {
+  if (gpu_malloc(&a, alloc, &ctx->rb) != hipSuccess) return fail(ctx, LBM_ERR_NOMEM, "access copy: hipMalloc failed");
+  if (gpu_malloc(&b, alloc, &ctx->rb) != hipSuccess) {
     (void)hipFree(a);
     return fail(ctx, LBM_ERR_NOMEM, "access copy: hipMalloc failed");
   }
@@ -2124,7 +2124,7 @@ FieldsView batch_view(lbm_batch* b) {
 template <typename T>
 int batch_upload(lbm_batch* b, T** dst, const std::vector<T>& src) {
   const size_t bytes = std::max<size_t>(1, src.size()) * sizeof(T);
-  HIPCHK(b->ctx, hipMalloc((void**)dst, bytes));
+  HIPCHK(b->ctx, gpu_malloc(dst, bytes, &b->ctx->rb));
   if (!src.empty())
     HIPCHK(b->ctx, hipMemcpyAsync(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice, b->ctx->stream));
   HIPCHK(b->ctx, hipStreamSynchronize(b->ctx->stream));
@@ -2298,10 +2298,10 @@ int lbm_batch_run_span(lbm_batch* b, int steps, int use_graph, double* torque) {
     if (b->ring) (void)hipFree(b->ring);
     b->ring = nullptr;
     b->ring_cap = 0;
-    HIPCHK(b->ctx, hipMalloc(&b->ring, (size_t)steps * K * ibm_ring_entry_bytes()));
+    HIPCHK(b->ctx, gpu_malloc(&b->ring, (size_t)steps * K * ibm_ring_entry_bytes(), &b->ctx->rb));
     b->ring_cap = (uint32_t)steps;
   }
-  if (b->ibm && !b->ring_pos) HIPCHK(b->ctx, hipMalloc((void**)&b->ring_pos, 256));
+  if (b->ibm && !b->ring_pos) HIPCHK(b->ctx, gpu_malloc(&b->ring_pos, 256, &b->ctx->rb));
   if (b->ibm) HIPCHK(b->ctx, launch_fill_f32((float*)b->ring_pos, 2, 0.0f, s));  // slot, blocks done
   int k = 0;
   if (use_graph && steps >= 2) {
@@ -2363,7 +2363,7 @@ int lbm_autotune_tiles(lbm_fields* fl, int trial_steps, uint32_t zb_out[2], doub
   hipStream_t s = fl->ctx->stream;
   // trial steps run on a copy of the populations: the state is untouched
   void* copy = nullptr;
-  if (hipMalloc(&copy, fl->f_bytes) != hipSuccess) return fail(fl->ctx, LBM_ERR_NOMEM, "autotune copy");
+  if (gpu_malloc(&copy, fl->f_bytes, &fl->ctx->rb) != hipSuccess) return fail(fl->ctx, LBM_ERR_NOMEM, "autotune copy");
   hipEvent_t ev[2 * 64 + 1] = {};
   const int T = std::min(trial_steps, 64) & ~1;  // whole even/odd pairs
   hipError_t err = hipMemcpyAsync(copy, fl->f_alloc, fl->f_bytes, hipMemcpyDeviceToDevice, s);
@@ -2464,7 +2464,7 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, uint32_t* best_grid, doubl
   };
   for (size_t j = 0; j < K; ++j) {
     lbm_fields* fl = b->mem[j];
-    if (hipMalloc(&copies[j], fl->f_bytes) != hipSuccess) {
+    if (gpu_malloc(&copies[j], fl->f_bytes, &b->ctx->rb) != hipSuccess) {
       release();
       return fail(b->ctx, LBM_ERR_NOMEM, "autotune copy of member %zu", j);
     }
@@ -2477,7 +2477,7 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, uint32_t* best_grid, doubl
     tab.push_back(a);
   }
   HydroArgs* dtab = nullptr;
-  if (hipMalloc((void**)&dtab, K * sizeof(HydroArgs)) != hipSuccess ||
+  if (gpu_malloc(&dtab, K * sizeof(HydroArgs), &b->ctx->rb) != hipSuccess ||
       hipMemcpyAsync(dtab, tab.data(), K * sizeof(HydroArgs), hipMemcpyHostToDevice, s) != hipSuccess) {
     release();
     if (dtab) (void)hipFree(dtab);
@@ -2704,10 +2704,8 @@ int lbm_adjoint_torque(lbm_fields* fl, int steps, int window, int snapshots, dou
     // zeroed: lamA, the force adjoints, omega_bar, the rotation rate's
     const size_t nz = Q * N + 9 * N + N + 1;
     const size_t bytes = (slots + 1) * (fb + lb) + lb + 256 + up(nz * sizeof(double)) + Q * N * sizeof(double);
-    if (hipMalloc((void**)&slab, bytes) != hipSuccess) {
-      slab = nullptr;
+    if (gpu_malloc(&slab, bytes, &fl->ctx->rb) != hipSuccess)
       return fail(fl->ctx, LBM_ERR_NOMEM, "adjoint workspace of %zu bytes (%zu snapshots)", bytes, slots + 1);
-    }
     char* at = slab;
     auto take = [&](size_t b) {
       char* p = at;

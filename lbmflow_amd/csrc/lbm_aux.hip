@@ -841,7 +841,7 @@ static void marker_stencil(const double p[3], const uint32_t dims[3], int radius
 template <typename T>
 static hipError_t upload(T** dst, const std::vector<T>& src) {
   const size_t bytes = std::max<size_t>(1, src.size()) * sizeof(T);
-  hipError_t e = hipMalloc((void**)dst, bytes);
+  hipError_t e = gpu_malloc(dst, bytes);
   if (e != hipSuccess) return e;
   if (!src.empty()) e = hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice);
   return e;
@@ -849,7 +849,7 @@ static hipError_t upload(T** dst, const std::vector<T>& src) {
 
 template <typename T>
 static hipError_t scratch(T** dst, size_t n) {
-  return hipMalloc((void**)dst, std::max<size_t>(1, n) * sizeof(T));
+  return gpu_malloc(dst, std::max<size_t>(1, n) * sizeof(T));
 }
 
 void ibm_destroy(IbmState* s) {

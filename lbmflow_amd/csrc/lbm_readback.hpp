@@ -51,6 +51,15 @@ class Readback {
     if (work_) (void)hipFree(work_);
   }
 
+  // Gives the device workspace back (no read is running); whether there was one.
+  bool release_work() {
+    const bool had = work_ != nullptr;
+    if (had) (void)hipFree(work_);
+    work_ = nullptr;
+    work_bytes_ = 0;
+    return had;
+  }
+
   // `planes` planes of n floats to out(plane).  produce(i0, cnt, w) enqueues on
   // `s` what writes the values i0 .. i0 + cnt - 1 of each plane to w + plane *
   // cnt.  hipErrorOutOfMemory: no workspace could be had.
@@ -252,8 +261,8 @@ class Readback {
   void* work(size_t want, size_t* have) {
     want = std::min(std::max(want, kMinWorkBytes), kWorkBytes);
     if (work_bytes_ < want) {
-      if (work_) (void)hipFree(work_);
-      for (work_ = nullptr, work_bytes_ = want; hipMalloc(&work_, work_bytes_) != hipSuccess;) {
+      (void)release_work();
+      for (work_bytes_ = want; hipMalloc(&work_, work_bytes_) != hipSuccess;) {
         (void)hipGetLastError();
         work_ = nullptr;
         if (work_bytes_ <= kMinWorkBytes) {
@@ -273,5 +282,20 @@ class Readback {
   void* work_ = nullptr;
   size_t work_bytes_ = 0;
 };
+
+// hipMalloc for every array of the library.  What the read-back keeps is given
+// back before an allocation is refused.  The runtime holds a refusal for the next
+// hipGetLastError, where it would be taken for a launch's: it is cleared here and
+// reported by the caller alone.
+template <typename T>
+inline hipError_t gpu_malloc(T** p, size_t bytes, Readback* rb = nullptr) {
+  hipError_t e = hipMalloc((void**)p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (rb && rb->release_work() && (e = hipMalloc((void**)p, bytes)) != hipSuccess) (void)hipGetLastError();
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
 
 }  // namespace lbm

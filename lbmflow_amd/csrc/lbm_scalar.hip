@@ -193,10 +193,10 @@ ScalarState* scalar_create(const FieldsView& v, double diffusivity, int Qs, std:
   s->ps = (N + 255) / 256 * 256;
   if (s->ps / 256 % 2 == 0) s->ps += 256;
   const size_t bytes = (size_t)Qs * s->ps * 4;
-  hipError_t e = hipMalloc((void**)&s->h, bytes);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->h2, bytes);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->C, N * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->partials, 6 * s->npartials * sizeof(double));
+  hipError_t e = gpu_malloc(&s->h, bytes, v.rb);
+  if (e == hipSuccess) e = gpu_malloc(&s->h2, bytes, v.rb);
+  if (e == hipSuccess) e = gpu_malloc(&s->C, N * 4, v.rb);
+  if (e == hipSuccess) e = gpu_malloc(&s->partials, 6 * s->npartials * sizeof(double), v.rb);
   if (e == hipSuccess) e = hipMemsetAsync(s->h, 0, bytes, v.stream);
   if (e == hipSuccess) e = hipMemsetAsync(s->h2, 0, bytes, v.stream);
   if (e == hipSuccess) e = hipMemsetAsync(s->C, 0, N * 4, v.stream);
@@ -259,8 +259,8 @@ int scalar_set(const FieldsView& v, ScalarState* s, const float* conc) {
   int rc = restore_partner(v, s);
   if (rc) return rc;
   float *dc = nullptr, *mom = nullptr;
-  AUXCHK(v, hipMalloc((void**)&dc, N * 4));
-  hipError_t e = hipMalloc((void**)&mom, 4 * N * 4);
+  AUXCHK(v, gpu_malloc(&dc, N * 4, v.rb));
+  hipError_t e = gpu_malloc(&mom, 4 * N * 4, v.rb);
   if (e == hipSuccess) e = hipMemcpyAsync(dc, conc, N * 4, hipMemcpyHostToDevice, v.stream);
   if (e == hipSuccess)
     e = launch_moments(v.Q, v.storage, v.parity, v.d, v.f, v.mask, v.F_mom, v.hp, 0, v.d.N, mom, mom + N,

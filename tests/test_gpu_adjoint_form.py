@@ -155,3 +155,17 @@ def test_gradient_leaves_the_state_of_the_forward_steps(snapshots):
             assert np.array_equal(x, y)
     a.close()
     b.close()
+
+
+def test_a_gradient_refused_for_memory_leaves_the_solver_usable():
+    """6,000 snapshots of a 96^3 tank do not fit any card: the call says so,
+    and the next one is not blamed for it."""
+    tc = cases.tank_case(96, nu=0.01, collision="trt", Q=19)
+    s = L.Solver(19, (96,) * 3, nu=0.01, collision="trt", solid=tc["solid"])
+    s.set_rotating_body(tc["pos"], tc["w"], tc["c"], (0.0, 0.0, tc["omega"]))
+    with pytest.raises(L.LbmError) as e:
+        s.adjoint_torque(6000, 10, 5999)
+    assert e.value.code == -4
+    s.run_with_ibm(2)
+    assert s.time == 2
+    s.close()

@@ -16,11 +16,12 @@ enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 typedef void* hipStream_t;
 typedef int* hipEvent_t;
 enum { hipMemcpyDeviceToHost, hipEventDisableTiming, hipHostMallocDefault };
+inline hipError_t last = hipSuccess;
 struct Pool {
   size_t used = 0, limit = ~(size_t)0;
   std::map<void*, size_t> held;
   hipError_t get(void** p, size_t n) {
-    if (used + n > limit) return hipErrorOutOfMemory;
+    if (used + n > limit) return last = hipErrorOutOfMemory;
     *p = malloc(n);
     held[*p] = n;
     used += n;
@@ -46,7 +47,11 @@ inline hipError_t hipEventDestroy(hipEvent_t e) { --events; delete e; return hip
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+inline hipError_t hipGetLastError() {
+  const hipError_t e = last;
+  last = hipSuccess;
+  return e;
+}
 """
 
 MAIN = r"""
@@ -104,6 +109,20 @@ int main() {
     Readback few;
     CHECK(read_ok(few, 105, 4) && pinned.used > 0 && read_ok(few, 3000001, 4) && read_ok(few, 105, 4));
   }
+  CHECK(dev.used == 0 && pinned.used == 0 && events == 0);
+  {
+    Readback rb;  // an allocation takes back what the read-back keeps; a refused one leaves no error behind
+    pinned.limit = ~(size_t)0;
+    CHECK(read_ok(rb, 9000001, 4) && dev.used == 64 * MiB);
+    dev.limit = 70 * MiB;
+    float *p = nullptr, *q = nullptr;
+    CHECK(lbm::gpu_malloc(&p, 32 * MiB, &rb) == hipSuccess && dev.used == 32 * MiB);
+    CHECK(lbm::gpu_malloc(&q, 64 * MiB, &rb) == hipErrorOutOfMemory && q == nullptr);
+    CHECK(lbm::gpu_malloc(&q, 64 * MiB) == hipErrorOutOfMemory && q == nullptr);
+    CHECK(read_ok(rb, 9000001, 4) && dev.used <= 70 * MiB);
+    hipFree(p);
+  }
+  CHECK(last == hipSuccess);
   CHECK(dev.used == 0 && pinned.used == 0 && events == 0);
   return 0;
 }
