@@ -494,19 +494,20 @@ bool wale_in_step(const lbm_fields* fl) {
 // keeps long runs; 16-bit even steps, whose tile is one line per plane, are
 // best nearly undealt.  The 256^3 D3Q27 fp32 tank (1.81 GB) is even either way
 // (1.157, 1.163 ms per pair), which is where the fp32 line lies.
-uint32_t hydro_deal(const lbm_fields* fl) {
+uint32_t hydro_deal(const lbm_fields* fl, int odd) {
   const size_t elem = fl->storage == kF32 ? 4 : 2;
   const size_t bytes = (size_t)fl->Q * fl->d.N * elem;
   if (bytes < (elem == 4 ? (size_t)1850000000 : (size_t)1000000000)) return kXcdStretch;
-  if (elem == 4) return fl->parity ? 8 : 9;  // 256, 512 blocks
-  return fl->parity ? 8 : 3;
+  if (elem == 4) return odd ? 8 : 9;  // 256, 512 blocks
+  return odd ? 8 : 3;
 }
 
-HydroArgs hydro_args(lbm_fields* fl) {
+// arguments of the step from the state of parity `odd`
+HydroArgs hydro_args(lbm_fields* fl, int odd) {
   HydroArgs a{};
   a.d = fl->d;
   a.t = fl->t;
-  a.tiles = fl->parity ? fl->tiles_odd : fl->tiles;
+  a.tiles = odd ? fl->tiles_odd : fl->tiles;
   a.ntiles = fl->ntiles;
   a.nseg = (fl->d.nx + 63) / 64;
   a.f = fl->f;
@@ -520,12 +521,14 @@ HydroArgs hydro_args(lbm_fields* fl) {
   a.F_cur = fl->F_cur;
   a.open = fl->open_face_cells ? 1 : 0;
   a.lin = fl->tiles_linear ? 1 : 0;
-  a.deal = hydro_deal(fl);
+  a.deal = hydro_deal(fl, odd);
   if (wale_in_step(fl))
     a.wale = WaleStep{fl->wale_work, fl->wale_work + 3 * fl->wale_ps, fl->wale_ps, fl->omega, fl->wale_cw2,
                       (float)wale_nu(fl), fl->wale_nut_max};
   return a;
 }
+
+HydroArgs hydro_args(lbm_fields* fl) { return hydro_args(fl, fl->parity); }
 
 // one device array to caller memory
 int read_array(lbm_fields* fl, void* dst, const void* src, size_t bytes) {
@@ -2364,9 +2367,15 @@ int lbm_autotune_tiles(lbm_fields* fl, int trial_steps, uint32_t zb_out[2], doub
   // trial steps run on a copy of the populations: the state is untouched
   void* copy = nullptr;
   if (gpu_malloc(&copy, fl->f_bytes, &fl->ctx->rb) != hipSuccess) return fail(fl->ctx, LBM_ERR_NOMEM, "autotune copy");
+  // with the closure inside the step its kernel is timed, on the state's own
+  // velocities (a work array), writing a scratch omega field; the plain kernel
+  // where the card has no room for that
+  float* omega = nullptr;
+  if (wale_in_step(fl)) (void)gpu_malloc(&omega, (size_t)fl->d.N * 4, &fl->ctx->rb);
   hipEvent_t ev[2 * 64 + 1] = {};
   const int T = std::min(trial_steps, 64) & ~1;  // whole even/odd pairs
   hipError_t err = hipMemcpyAsync(copy, fl->f_alloc, fl->f_bytes, hipMemcpyDeviceToDevice, s);
+  if (err == hipSuccess && omega) err = launch_wale_local(fl->Q, fl->storage, wale_fields(fl), nullptr, s);
   for (int k = 0; k <= T && err == hipSuccess; ++k) err = hipEventCreate(&ev[k]);
   static const uint32_t cand_even[] = {1, 2, 4, 8, 16, 32};
   static const uint32_t cand_odd[] = {1, 4, 8, 16, 32, 64};
@@ -2380,22 +2389,24 @@ int lbm_autotune_tiles(lbm_fields* fl, int trial_steps, uint32_t zb_out[2], doub
     fl->zb_set[1] = cand_odd[c];
     rc = rebuild_tiles(fl);
     if (rc) break;
-    HydroArgs a = hydro_args(fl);
-    a.f = (char*)copy + off;
-    a.wale = WaleStep{};  // a trial writes no omega field
+    HydroArgs args[2];  // each parity under its own order and dealing
+    for (int p = 0; p < 2; ++p) {
+      args[p] = hydro_args(fl, p);
+      args[p].f = (char*)copy + off;
+      if (!omega) args[p].wale = WaleStep{};
+      args[p].wale.omega = omega;
+    }
     const int p0 = fl->parity;
     double sum[2] = {0.0, 0.0};
     // one untimed pair, then T launches with an event between each
     for (int t = 0; t < 2 && err == hipSuccess; ++t) {
       const int p = (p0 + t) & 1;
-      a.tiles = p ? fl->tiles_odd : fl->tiles;
-      err = launch_hydro(fl->Q, fl->storage, fl->collision, p, a, s);
+      err = launch_hydro(fl->Q, fl->storage, fl->collision, p, args[p], s);
     }
     if (err == hipSuccess) err = hipEventRecord(ev[0], s);
     for (int t = 0; t < T && err == hipSuccess; ++t) {
       const int p = (p0 + t) & 1;
-      a.tiles = p ? fl->tiles_odd : fl->tiles;
-      err = launch_hydro(fl->Q, fl->storage, fl->collision, p, a, s);
+      err = launch_hydro(fl->Q, fl->storage, fl->collision, p, args[p], s);
       if (err == hipSuccess) err = hipEventRecord(ev[t + 1], s);
     }
     if (err == hipSuccess) err = hipEventSynchronize(ev[T]);
@@ -2417,6 +2428,7 @@ int lbm_autotune_tiles(lbm_fields* fl, int trial_steps, uint32_t zb_out[2], doub
   for (int k = 0; k <= T; ++k)
     if (ev[k]) (void)hipEventDestroy(ev[k]);
   (void)hipFree(copy);
+  if (omega) (void)hipFree(omega);
   if (err != hipSuccess && !rc) rc = fail(fl->ctx, LBM_ERR_DEVICE, "autotune trial: %s", hipGetErrorString(err));
   if (rc) {
     fl->zb_set[0] = keep[0];

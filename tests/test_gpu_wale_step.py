@@ -80,14 +80,21 @@ def test_body_and_riding_scalar(storage):
             assert np.array_equal(x, y)
 
 
-def test_tiles_autotuned_under_the_closure_leave_the_field():
-    s, fl = cavity(27, "cm", "f32", (64, 12, 11))
-    s.set_wale(True)
-    s.run(3)
+@pytest.mark.parametrize("storage,dims,steps", [("f32", (64, 12, 11), 3), ("f16", (19, 13, 9), 2)])
+def test_tiles_autotuned_under_the_closure_leave_the_field(storage, dims, steps):
+    s, fl = cavity(27, "cm", storage, dims)
+    b, _ = cavity(27, "cm", storage, dims)
+    for v in (s, b):
+        v.set_wale(True)
+        v.run(steps)
     om, f = s.omega_field(), s.populations()
     s.autotune_tiles(4)
     assert np.array_equal(s.omega_field(), om) and np.array_equal(s.populations(), f)
+    for v in (s, b):
+        v.run(3)
+    assert np.array_equal(s.omega_field(), b.omega_field()) and np.array_equal(s.populations(), b.populations())
     s.close()
+    b.close()
 
 
 def test_calls_without_a_step_leave_the_field():
