@@ -247,8 +247,14 @@ hipError_t launch_adj_collide_stream(int storage, int odd, const Dom& d, const v
                                      const HydroParams& p, const uint32_t* flist, uint32_t nlist, const double* lam_in,
                                      double* lam_out, double* omega_bar, double* Fbar, double* Gout,
                                      hipStream_t s) {
+  // One stretch per XCD below 1 GB of the pass's bytes (about 400 per cell),
+  // short runs above (xcd_remap).  us per pass of a tank, stretch -> dealt, medians
+  // of four processes: 96^3 64.2 -> 63.5, 112^3 104.3 -> 107.0, 128^3 (0.84 GB) 155
+  // -> 165, 144^3 (1.19 GB) 223.5 -> 218.4, 160^3 301 -> 292, 192^3 499 -> 483,
+  // 224^3 777 -> 753, 256^3 1132 -> 1157 (1130 +- 30 either way).
+  const uint32_t deal = (size_t)d.N * 400 < 1000000000 ? kXcdStretch : 5u;
   AdjArgs a{d, f, mask, omega, F_cur, F_mom, p, lam_in, lam_out, omega_bar, Fbar, Gout,
-            flist, F_cur && F_mom ? nlist : 0u, 5u};
+            flist, F_cur && F_mom ? nlist : 0u, deal};
   if (storage == kF32) return adj_s<float>(odd, a, s);
   if (storage == kF16) return adj_s<_Float16>(odd, a, s);
   return adj_s<bf16s>(odd, a, s);

@@ -492,12 +492,24 @@ bool wale_in_step(const lbm_fields* fl) {
 //   384 x 256 x 256 periodic D3Q27 fp16  0.591 / 0.717 -> 0.515 / 0.721
 // The odd step's x-shifted rows share lines between neighbouring tiles, so it
 // keeps long runs; 16-bit even steps, whose tile is one line per plane, are
-// best nearly undealt.  The 256^3 D3Q27 fp32 tank (1.81 GB) is even either way
-// (1.157, 1.163 ms per pair), which is where the fp32 line lies.
+// best nearly undealt.
+// Where the lines lie, closed cavities, even / odd ms, stretch -> dealt:
+//   fp32 D3Q19 1.28 GB  0.504 / 0.524 -> 0.514 / 0.540
+//        D3Q27 1.49     0.609 / 0.677 -> 0.610 / 0.663
+//        D3Q27 1.81     0.724 / 0.769 -> 0.737 / 0.798  (256^3)
+//        D3Q19 1.82     0.731 / 0.763 -> 0.729 / 0.753
+//        D3Q27 1.99     0.819 / 0.867 -> 0.813 / 0.856
+//        D3Q19 2.49     1.005 / 1.120 -> 0.992 / 1.049
+//   between 1.5 and 2 GB the two are within 2 % but for the power of two, which
+//   the line leaves to the stretch.
+// 16-bit, whole step of a tank with a body, stretch -> dealt ms: D3Q27 0.75 GB
+// 0.349 -> 0.352, D3Q19 0.76 GB 0.363 -> 0.351, D3Q27 0.91 GB 0.436 -> 0.414.
+// Below, tanks lose and cavities gain (0.61 GB launch 0.241 -> 0.244, 0.298 ->
+// 0.287), boxes on linear tiles lose (0.28 GB 0.134 -> 0.147).
 uint32_t hydro_deal(const lbm_fields* fl, int odd) {
   const size_t elem = fl->storage == kF32 ? 4 : 2;
   const size_t bytes = (size_t)fl->Q * fl->d.N * elem;
-  if (bytes < (elem == 4 ? (size_t)1850000000 : (size_t)1000000000)) return kXcdStretch;
+  if (bytes < (elem == 4 ? (size_t)1850000000 : (size_t)750000000)) return kXcdStretch;
   if (elem == 4) return odd ? 8 : 9;  // 256, 512 blocks
   return odd ? 8 : 3;
 }

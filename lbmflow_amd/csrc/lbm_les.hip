@@ -269,7 +269,14 @@ static uint32_t wale_zlen(const Dom& d) {
 template <int Q, typename S>
 static void local_q(const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
   const dim3 grid((a.d.N + 255) / 256), block(256);
-  const uint32_t deal = a.d.N < (1u << 24) ? kXcdStretch : 5u;
+  // One stretch per XCD while populations, mask and the six planes fit the
+  // last-level cache (256 MiB), short runs beyond (xcd_remap).  Whole step of a
+  // closed D3Q27 cavity, stretch -> dealt ms: fp16 144^3 (245 MB) 0.1455 -> 0.1472,
+  // 152^3 (288) 0.1864 -> 0.1833, 192^3 0.405 -> 0.388; fp32 128^3 (285) 0.1458 ->
+  // 0.1460, with a tracer taken along 0.172 -> 0.174, 136^3 (342) 0.182 -> 0.179,
+  // 192^3 0.604 -> 0.578, 320^3 2.875 -> 2.867.
+  const size_t bytes = ((size_t)Q * sizeof(S) + 28) * a.d.N;
+  const uint32_t deal = bytes < 270000000 ? kXcdStretch : 5u;
   const ScalarStepArgs none{};
   if (sc)
     hipLaunchKernelGGL((k_wale_local<Q, S, false, 7>), grid, block, 0, s, a, deal, *sc);

@@ -364,7 +364,14 @@ int scalar_step(const FieldsView& v, ScalarState* s) {
   ScalarStepArgs st;
   int rc = scalar_turn(v, s, &st);
   if (rc) return rc;
-  const VelArgs a{v.d, v.f, v.mask, v.F_mom, v.hp, v.parity, v.d.N < (1u << 24) ? kXcdStretch : 5u};
+  // One stretch per XCD while the last-level cache holds most of what the pass
+  // reads, short runs beyond (xcd_remap).  Whole step of a closed cavity, stretch
+  // -> dealt ms: D3Q7 144^3 fp16 D3Q27 (257 MB read) 0.144 -> 0.147, fp32 D3Q19
+  // (322) 0.162 -> 0.167, 160^3 (352, 442) 0.214 -> 0.209 and 0.265 -> 0.253;
+  // hydro lattice 128^3 (327, 348) 0.173 -> 0.178 and 0.216 -> 0.220, 144^3 (466,
+  // 495) 0.276 -> 0.266 and 0.302 -> 0.292; 320^3 and more within 1 %.
+  const size_t reads = ((size_t)v.Q * (v.storage == kF32 ? 4 : 2) + 4 + 4 * (size_t)s->Qs) * v.d.N;
+  const VelArgs a{v.d, v.f, v.mask, v.F_mom, v.hp, v.parity, reads < 350000000 ? kXcdStretch : 5u};
   if (v.storage == kF32)
     scalar_step_s<float>(v.Q, s->Qs, a, st, v.stream);
   else if (v.storage == kF16)
