@@ -1,7 +1,9 @@
 """The adjoint collide-stream kernel over the forms it accepts: periodic axes,
-16-bit storage, BGK, obstacles with walls on every side and forced cells in
-wall-linked places, against finite differences of J with respect to the
-per-cell viscosity (the test of test_gpu_adjoint at other domains)."""
+BGK, obstacles with walls on every side and forced cells in wall-linked places,
+against finite differences of J with respect to the per-cell viscosity (the
+test of test_gpu_adjoint at other domains); 16-bit storage against the fp32
+gradient from the same state; the largest domains; and what the call leaves
+behind."""
 import numpy as np
 import pytest
 
@@ -58,6 +60,51 @@ def test_directional_gradient_matches_differences(collision, periodic, dims):
     ad = float(np.dot(a["dJ_dnu"], d))
     # fp32 forward: J carries about 1e-7 of rounding against steps of 1e-2
     assert abs(ad - fd) <= 2e-3 * abs(fd) + 1e-5 * abs(a["J"])
+
+
+@pytest.mark.parametrize("storage,eps", [("f16", 2.0 ** -11), ("bf16", 2.0 ** -8)])
+@pytest.mark.parametrize("before", [2, 3])  # the state's parity
+@pytest.mark.parametrize("periodic", [(0, 0, 0), (1, 1, 1)])
+def test_sixteen_bit_gradient_from_an_exact_state(storage, eps, before, periodic):
+    """Two steps from a 16-bit state, and from the same values held in fp32.
+    With the torque of the second step alone the viscosity acts in the first,
+    whose populations are the same numbers in both, so that the gradients differ
+    by how the second step's rounded velocities and densities enter the body's
+    update: a few units of the storage's last place."""
+    dims = nx, ny, nz = 21, 16, 13
+    solid = np.zeros((nz, ny, nx), np.uint8)
+    if not periodic[0]:
+        for ax in range(3):
+            for k in (0, -1):
+                ix = [slice(None)] * 3
+                ix[ax] = k
+                solid[tuple(ix)] = 1
+    solid[3:6, 4:6, 5:7] = 1
+    rng = np.random.RandomState(7)
+    c = np.array([nx / 2.0, ny / 2.0, nz / 2.0])
+    pos = c + rng.uniform(-3.0, 3.0, (30, 3))
+    nu = 0.05 * (1.0 + 0.2 * rng.rand(nx * ny * nz))
+    rho, u = cases.tgv_field(dims, 0.02)
+
+    def solver(st):
+        s = L.Solver(19, dims, nu=0.05, collision="trt", storage=st, periodic=periodic, solid=solid.reshape(-1))
+        s.set_omega_field((1.0 / (3.0 * nu + 0.5)).astype(np.float32))
+        return s
+
+    a, b = solver(storage), solver("f32")
+    a.init_with(rho, u)
+    a.run(before)
+    b.set_populations(a.populations())
+    out = []
+    for s in (a, b):
+        s.set_rotating_body(pos, 0.3 * np.ones(30), c, (0.0, 0.0, 0.012))
+        out.append(s.adjoint_torque(2, 1, 2))
+        s.close()
+    x, y = out
+    for k in ("J", "dJ_domega"):
+        assert abs(x[k] - y[k]) <= 8 * eps * abs(y[k])
+    d = x["dJ_dnu"] - y["dJ_dnu"]
+    assert np.linalg.norm(y["dJ_dnu"]) > 0.0 and np.linalg.norm(d) <= 8 * eps * np.linalg.norm(y["dJ_dnu"])
 
 
 def test_domain_beyond_the_lane_offset_is_refused():
