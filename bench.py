@@ -423,7 +423,7 @@ def workload_surface(args):
 
 
 def workload_batch(args):
-    """64 tanks in one persistent launch (edges U[48,160], tip U[0.02,0.06],
+    """64 tanks in one launch (edges U[48,160], tip U[0.02,0.06],
     nu U[0.002,0.02], D3Q19 TRT fp32), graph-captured step, autotuned grid."""
     import lbmflow_amd as L
 
@@ -594,8 +594,9 @@ def workload_channel(args):
 
 def workload_les(args):
     """The 512^3 tank step with the WALE closure recomputed on the device
-    before every collision (moments, WALE omega field, collide-stream with
-    that field); reports the step rate and the closure's share of it."""
+    before every collision (a velocity and strain pass, then the closure inside
+    the collide-stream kernel); reports the step rate and the closure's share
+    of it."""
     cfg = tank_config(args.size)
     Q = args.lattice
     s, n_markers = build_gpu(cfg, args.storage, args.collision, Q)
@@ -611,14 +612,13 @@ def workload_les(args):
     ms, ms0 = 1e3 * dt / args.steps, 1e3 * dt0 / args.steps
     S = STORAGE_BYTES[args.storage]
     # the closure's algorithmic bytes: per fluid cell the local pass reads Q
-    # populations and the mask and writes the velocity and 3 strain
-    # components, the gradient pass reads the mask, the cell's velocity and
-    # strain and writes omega (neighbour velocities come from L2); per solid
-    # cell the local pass reads the mask and writes 6 zeros, the gradient pass
-    # reads the mask and writes omega
+    # populations and the mask and writes the velocity and 3 strain components,
+    # the collide-stream kernel reads the velocity and the strain (neighbour
+    # velocities come from L2) and writes omega; per solid cell the local pass
+    # reads the mask
     n_total = args.size ** 3
-    b_cell = (Q * S + 4 + 24) + (4 + 24 + 4)
-    b_solid = (4 + 24) + (4 + 4)
+    b_cell = (Q * S + 4 + 24) + (24 + 4)
+    b_solid = 4
     closure_bytes = fluid * b_cell + (n_total - fluid) * b_solid
     wale_ms = ms - ms0
     print(f"[bench] les: {ms:.3f} ms/step (plain {ms0:.3f}), closure {wale_ms:.3f} ms, "

@@ -401,7 +401,7 @@ int lbm_ibm_torque_integral(lbm_fields* fl, int reset, double out[4]);
  * another through the runner (crates/lbm-cli/src/sweep.rs:61-106, grid
  * expansion crates/lbm-scenario/src/sweep.rs:52-71).  A batch steps several
  * independent closed domains (same lattice, storage and collision kind; each
- * with its own grid, masks, rates and rotating body) together: one persistent
+ * with its own grid, masks, rates and rotating body) together: one
  * collide-stream launch over their concatenated tile lists, one forced-cell
  * launch, one set of IBM launches for all bodies.  Members must not be
  * changed while a batch over them exists; the batch checks this. */
@@ -409,13 +409,14 @@ typedef struct lbm_batch lbm_batch;
 int lbm_batch_create(lbm_ctx* ctx, lbm_fields* const* members, int n, lbm_batch** out);
 void lbm_batch_destroy(lbm_batch* b);
 int lbm_batch_info(const lbm_batch* b, int* members, uint32_t* tiles, uint32_t* forced_cells, uint32_t* grid);
-/* Persistent grid (workgroups of 256) of the collide-stream launch. */
+/* Grid (workgroups of 256) of the collide-stream launch: by default one wave
+ * per tile, a smaller one strides over the tiles. */
 int lbm_batch_set_grid(lbm_batch* b, uint32_t grid);
 /* `steps` runner steps of every member (as lbm_run_ibm_span, or plain
  * collide-stream steps when the members have no rotating body).  torque
  * (nullable) receives members x steps x 3 values, member-major. */
 int lbm_batch_run_span(lbm_batch* b, int steps, int use_graph, double* torque);
-/* Times the collide-stream launch over a set of persistent grid sizes on
+/* Times the collide-stream launch over a set of grid sizes on
  * scratch copies of the populations (the members' state is untouched) and
  * keeps the fastest. */
 int lbm_batch_autotune(lbm_batch* b, int trial_steps, uint32_t* best_grid, double* best_ms);

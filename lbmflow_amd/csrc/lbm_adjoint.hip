@@ -49,7 +49,7 @@ struct AdjArgs {
 // and Lm = lam*_a - lam*_b, so the direct part, the feq and the S adjoints are
 // never stored: what lives through the kernel is lam* (19 f64) and f (19 fp32).
 // The form that held all three took 296 VGPRs, one wave per SIMD, and 240 us
-// on the 128^3 tank; this one 168, three waves, and 162 us (0.53 GB, 3.3 TB/s).
+// on the 128^3 tank; this one 168, three waves, and 155 us (0.53 GB, 3.4 TB/s).
 // Solid cells are skipped and their adjoint is left undefined: what a fluid
 // cell pulls from one is always replaced by its own reflected value.
 // FORCED cells (those of the force list) take the source's terms as well, in a

@@ -314,8 +314,13 @@ int rebuild_tiles(lbm_fields* fl) {
   // (zb = 1).  Odd steps write a row's slots from the row itself
   // (bounce-back) and from its upstream rows; keeping z-neighbour rows a
   // few tiles apart lets one XCD's L2 merge those writes into whole lines
-  // before they reach memory (512^3 D3Q27 tank, odd step: fp32 4.68 ms at
-  // zb = 1, 4.48 at zb = 32; fp16 3.71 at zb = 1, 3.11 at zb = 16).
+  // before they reach memory.  D3Q27 tanks, odd step, ms at zb = 1 / 4 / 8 / 16
+  // / 32: fp32 256^3 (one stretch per XCD, hydro_deal) 0.636 / 0.636 / 0.641 /
+  // 0.626 / 0.623, dealt 400^3 2.40 / 2.44 / 2.45 / 2.47 / 2.48, 512^3 4.05 / 4.04
+  // / 4.1 / 4.08 / 4.15; fp16, all dealt, 256^3 0.423 / 0.427 / 0.436 / 0.434 /
+  // 0.428, 400^3 1.376 / 1.378 / 1.371 / 1.371 / 1.382, 512^3 2.66 / 2.60 / 2.62 /
+  // 2.60 / 2.68.  The dealing took over most of what the order gained; within
+  // 3 % of the best here, the rest is lbm_autotune_tiles'.
   uint32_t zb_even = 1, zb_odd = fl->storage == kF32 ? 32 : 16;
   if (const char* e = getenv("LBM_TILE_ZBLOCK")) {  // "n" (both parities) or "even,odd"
     zb_even = zb_odd = (uint32_t)std::max(1, atoi(e));

@@ -909,10 +909,9 @@ __global__ __launch_bounds__(256) void k_hydro_list(HydroArgs a) {
 
 // ---------------------------------------------------------------------------
 // Batched domains: one launch walks the concatenated tile lists of K
-// independent (non-periodic) domains; entry e = (tile, domain).  Each wave
-// strides over entries (a persistent grid, or a grid of one entry per wave)
-// and reads its tile's domain arguments from the table (wave-uniform, so
-// scalar loads).
+// independent (non-periodic) domains; entry e = (tile, domain).  A wave takes
+// one entry, or strides over them when the grid was set smaller, and reads its
+// tile's domain arguments from the table (wave-uniform, so scalar loads).
 // ---------------------------------------------------------------------------
 template <int Q, typename S, int KIND, bool ODD>
 __global__ __launch_bounds__(256) void k_hydro_batch(const HydroArgs* __restrict__ tab,

@@ -86,7 +86,7 @@ struct HydroArgs {
   WaleStep wale;            // per-step closure inside the step (vel null: none)
   int open;                 // fluid on a non-periodic (open) face: wrap every offset
   uint32_t deal;            // how the tile blocks are dealt to the XCDs (xcd_remap)
-  int lin;                  // tiles are 64-cell blocks of the linear index (no axis wraps)
+  int lin;                  // tiles are 64-cell blocks of the linear index
 };
 
 // Open faces (lbm_open.hip): FaceBC kinds of params.rs:232-252, faces in

@@ -18,9 +18,9 @@
 // On closed domains the per-step closure does without the second pass: the
 // collide-stream kernel takes the same gradient and nu_t of each cell it
 // updates (lbm_wale.hpp).
-// Bytes per fluid cell: 4Q + 4 (mask) + 24 in the first pass; 4 + 24 + the
-// neighbours' velocities (mostly from L2) + 4 in the second, against two
-// full population reads for a moment pass followed by a strain pass.
+// Bytes per fluid cell: Q S + 4 (mask) + 24 in the first pass; 4 + 24 + the
+// neighbours' velocities (mostly from L2) + 4 in the second, 24 + 4 inside the
+// step.  Per solid cell 4 in the first pass (nothing is stored), 8 in the second.
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
 #include "lbm_scalar.hpp"

@@ -623,7 +623,7 @@ def mixing_time_from_cv(t, cv):
 
 
 class Batch:
-    """Several closed domains stepped together: one persistent collide-stream
+    """Several closed domains stepped together: one collide-stream
     launch over their concatenated tile lists and one set of IBM launches for
     all rotating bodies (lbm_batch_* in include/lbm_hip.h).  The member
     solvers keep their state and stay readable; they must not be changed
