@@ -110,9 +110,11 @@ class Readback {
       }
       if (one) {  // one slot, one wait, no thread
         size_t at = 0;
-        for (const Seg& g : segs) {
-          if (e == hipSuccess) e = hipMemcpyAsync(pin_ + at, g.src, g.bytes, hipMemcpyDeviceToHost, s);
-          at += g.bytes;
+        for (size_t a = 0, b; a < segs.size() && e == hipSuccess; a = b) {
+          size_t n = 0;
+          for (b = a; b < segs.size() && segs[b].src == (const char*)segs[a].src + n; ++b) n += segs[b].bytes;
+          e = hipMemcpyAsync(pin_ + at, segs[a].src, n, hipMemcpyDeviceToHost, s);
+          at += n;
         }
         const hipError_t w = hipStreamSynchronize(s);
         if (e == hipSuccess) e = w;
@@ -132,14 +134,31 @@ class Readback {
         } catch (...) {
         }
       }
+      // one copy per slot, over as many segments as lie together in the
+      // source: a copy costs the caller up to 45 us whatever its size (populations
+      // of 24^3 cells, 19 planes of 55 KB: 1.03 -> 0.07 ms)
+      Item it;
+      const char* src = nullptr;
+      size_t fill = 0;
+      auto flush = [&] {
+        if (fill == 0 || e != hipSuccess) return;
+        it.slot = job.take(pool.empty() ? this : nullptr);
+        e = hipMemcpyAsync(pin_ + (size_t)it.slot * kSlotBytes, src, fill, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(ev_[it.slot], s);
+        if (e == hipSuccess) job.put(it);
+        fill = 0;
+        it.parts = 0;
+      };
       for (const Seg& g : segs)
-        for (size_t at = 0; at < g.bytes && e == hipSuccess; at += kSlotBytes) {
-          const size_t n = std::min(kSlotBytes, g.bytes - at);
-          const int k = job.take(pool.empty() ? this : nullptr);
-          e = hipMemcpyAsync(pin_ + (size_t)k * kSlotBytes, (const char*)g.src + at, n, hipMemcpyDeviceToHost, s);
-          if (e == hipSuccess) e = hipEventRecord(ev_[k], s);
-          if (e == hipSuccess) job.put(Item{k, (char*)g.dst + at, n});
+        for (size_t at = 0, n; at < g.bytes && e == hipSuccess; at += n) {
+          const char* from = (const char*)g.src + at;
+          if (fill && (fill == kSlotBytes || it.parts == kParts || from != src + fill)) flush();
+          if (fill == 0) src = from;
+          n = std::min(kSlotBytes - fill, g.bytes - at);
+          it.part[it.parts++] = {(char*)g.dst + at, n};
+          fill += n;
         }
+      flush();
     }
     job.close();
     if (pool.empty()) worker(device, job);
@@ -150,10 +169,14 @@ class Readback {
   }
 
  private:
+  // a filled slot and where its contents go
+  static constexpr int kParts = 28;  // the populations' planes lie together
   struct Item {
-    int slot;
-    char* dst;
-    size_t bytes;
+    int slot = 0, parts = 0;
+    struct {
+      char* dst;
+      size_t bytes;
+    } part[kParts];
   };
   // free slots and filled ones, each at most kSlots: fixed arrays, so that no
   // thread allocates
@@ -207,10 +230,15 @@ class Readback {
 
   void drain(const Item& it, Job& job) {
     const hipError_t e = hipEventSynchronize(ev_[it.slot]);
-    if (e == hipSuccess)
-      memcpy(it.dst, pin_ + (size_t)it.slot * kSlotBytes, it.bytes);
-    else
+    if (e == hipSuccess) {
+      const char* from = pin_ + (size_t)it.slot * kSlotBytes;
+      for (int k = 0; k < it.parts; ++k) {
+        memcpy(it.part[k].dst, from, it.part[k].bytes);
+        from += it.part[k].bytes;
+      }
+    } else {
       job.err.store((int)e);
+    }
     {
       std::lock_guard<std::mutex> lk(job.mu);
       job.free[job.nfree++] = it.slot;

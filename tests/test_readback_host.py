@@ -1,6 +1,6 @@
 """The read-back object on the CPU: its header compiled against a stand-in for
 the runtime that counts device and pinned bytes and refuses them past a limit.
-Small reads hold what they need and no more, a card with little memory left is
+Small reads hold what they need and no more, planes go in few copies, a card with little memory left is
 read in small pieces, and reads without pinned memory or threads still work."""
 import os
 import subprocess
@@ -35,12 +35,16 @@ struct Pool {
   }
 };
 inline Pool dev, pinned;
-inline int events = 0;
+inline int events = 0, copies = 0;
 template <typename T> hipError_t hipMalloc(T** p, size_t n) { return dev.get((void**)p, n); }
 inline hipError_t hipFree(void* p) { return dev.put(p); }
 inline hipError_t hipHostMalloc(void** p, size_t n, int) { return pinned.get(p, n); }
 inline hipError_t hipHostFree(void* p) { return pinned.put(p); }
-inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+  ++copies;
+  memcpy(d, s, n);
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, int) { ++events; *e = new int; return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t e) { --events; delete e; return hipSuccess; }
@@ -61,7 +65,7 @@ using lbm::Readback;
 static int pieces;
 static bool read_ok(Readback& rb, uint32_t n, uint32_t planes) {
   std::vector<float> out((size_t)n * planes, -1.0f);
-  pieces = 0;
+  pieces = copies = 0;
   const hipError_t e = rb.read_planes(0, nullptr, n, planes, [&](uint32_t k) { return out.data() + (size_t)k * n; },
                                       [&](uint32_t i0, uint32_t cnt, float* w) {
     ++pieces;
@@ -82,8 +86,10 @@ int main() {
     Readback rb;  // small reads hold little, larger ones grow to the bounds
     CHECK(read_ok(rb, 105, 4) && dev.used <= MiB / 8 && pinned.used <= 2 * MiB && pieces == 1);
     CHECK(read_ok(rb, 32768, 27) && dev.used <= 4 * MiB && pieces == 1);
+    CHECK(copies == 2);  // planes that lie together go in one copy per slot
     CHECK(read_ok(rb, 9000001, 4) && dev.used == 64 * MiB && pinned.used == 48 * MiB && pieces == 3);
-    CHECK(read_ok(rb, 105, 27) && dev.used == 64 * MiB);
+    CHECK(copies <= 69 + 3);
+    CHECK(read_ok(rb, 105, 27) && dev.used == 64 * MiB && copies == 1);
   }
   CHECK(dev.used == 0 && pinned.used == 0 && events == 0);
   {
