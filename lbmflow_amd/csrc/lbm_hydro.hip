@@ -812,16 +812,23 @@ __device__ __forceinline__ void cell_step(const HydroArgs& a, uint32_t i, uint32
   }
 }
 
-template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool WALE>
+template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool LIN, bool WALE>
 __device__ __forceinline__ void hydro_tile(const HydroArgs& a) {
   // each wave takes one active 64-cell tile; tiles of only solid (or
   // force-listed) cells are never launched
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x, a.deal);
+  // What the tile entry's address needs is loaded at once: left to the compiler
+  // each side of the remap's branch waited for its own scalar loads, a second
+  // latency before the wave's first vector load.
+  uint32_t n = gridDim.x, deal = a.deal, ntiles = a.ntiles;
+  uint64_t list = (uint64_t)a.tiles;
+  asm volatile("" : "+s"(n), "+s"(deal), "+s"(ntiles), "+s"(list));
+  const auto* tiles = (const __attribute__((address_space(1))) uint32_t*)list;
+  const uint32_t b = xcd_remap(blockIdx.x, n, deal);
   const uint32_t t = b * 4 + (threadIdx.x >> 6);
-  if (t >= a.ntiles) return;
-  const uint32_t te = __builtin_amdgcn_readfirstlane(a.tiles[t]);  // one tile per wave
+  if (t >= ntiles) return;
+  const uint32_t te = __builtin_amdgcn_readfirstlane(tiles[t]);  // one tile per wave
   const uint32_t tile = te & kTileId;
-  if (a.lin) {
+  if (WRAP ? LIN : a.lin != 0) {
     // linear tile: cells 64 tile .. 64 tile + 63 across row ends (where no
     // axis wraps every neighbour shift is the linear one, elsewhere each lane
     // takes its own coordinates)
@@ -857,9 +864,13 @@ __device__ __forceinline__ void hydro_tile(const HydroArgs& a) {
   }
 }
 
-template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP>
+// WRAP with LIN: packed tiles on a wrapped domain, a kernel of their own.  Both
+// tile forms in one kernel took up to 18 VGPRs more (odd D3Q19 CM with a force 127
+// -> 137, a wave per SIMD fewer), which the row tiles paid for (periodic 256^3
+// D3Q27 fp32 with a force 0.774 against 0.759 ms).
+template <int Q, typename S, int KIND, bool ODD, bool FON, bool WRAP, bool LIN>
 __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
-  hydro_tile<Q, S, KIND, ODD, FON, WRAP, false>(a);
+  hydro_tile<Q, S, KIND, ODD, FON, WRAP, LIN, false>(a);
 }
 
 // The step with the WALE closure inside (closed domains, no uniform force):
@@ -875,7 +886,7 @@ __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
 // where nu_t's 380 VALU instructions per wave make it VALU-bound).
 template <int Q, typename S, int KIND, bool ODD>
 __global__ __launch_bounds__(256, 4) void k_hydro_wale(HydroArgs a) {
-  hydro_tile<Q, S, KIND, ODD, false, false, true>(a);
+  hydro_tile<Q, S, KIND, ODD, false, false, false, true>(a);
 }
 
 // Cells carrying a per-cell force: the velocity uses the force of the cached
@@ -968,6 +979,16 @@ __global__ __launch_bounds__(256) void k_hydro_list_batch(const HydroArgs* __res
 
 static inline uint32_t blocks_for(size_t n, uint32_t bs = 256) { return (uint32_t)((n + bs - 1) / bs); }
 
+template <int Q, typename S, int KIND, bool ODD, bool FON>
+static void hydro_w(bool wrap, const HydroArgs& a, dim3 grid, hipStream_t s) {
+  if (!wrap)
+    hipLaunchKernelGGL((k_hydro<Q, S, KIND, ODD, FON, false, false>), grid, dim3(256), 0, s, a);
+  else if (a.lin)
+    hipLaunchKernelGGL((k_hydro<Q, S, KIND, ODD, FON, true, true>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_hydro<Q, S, KIND, ODD, FON, true, false>), grid, dim3(256), 0, s, a);
+}
+
 template <int Q, typename S, int KIND>
 static hipError_t hydro_q(int odd, const HydroArgs& a, hipStream_t s, bool list) {
   if (list) {
@@ -996,17 +1017,10 @@ static hipError_t hydro_q(int odd, const HydroArgs& a, hipStream_t s, bool list)
       hipLaunchKernelGGL((k_hydro_wale<Q, S, KIND, false>), grid, block, 0, s, a);
     return hipGetLastError();
   }
-  const int sel = (odd ? 4 : 0) | (fon ? 2 : 0) | (wrap ? 1 : 0);
-  switch (sel) {
-    case 0: hipLaunchKernelGGL((k_hydro<Q, S, KIND, false, false, false>), grid, block, 0, s, a); break;
-    case 1: hipLaunchKernelGGL((k_hydro<Q, S, KIND, false, false, true>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_hydro<Q, S, KIND, false, true, false>), grid, block, 0, s, a); break;
-    case 3: hipLaunchKernelGGL((k_hydro<Q, S, KIND, false, true, true>), grid, block, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((k_hydro<Q, S, KIND, true, false, false>), grid, block, 0, s, a); break;
-    case 5: hipLaunchKernelGGL((k_hydro<Q, S, KIND, true, false, true>), grid, block, 0, s, a); break;
-    case 6: hipLaunchKernelGGL((k_hydro<Q, S, KIND, true, true, false>), grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL((k_hydro<Q, S, KIND, true, true, true>), grid, block, 0, s, a); break;
-  }
+  if (odd)
+    fon ? hydro_w<Q, S, KIND, true, true>(wrap, a, grid, s) : hydro_w<Q, S, KIND, true, false>(wrap, a, grid, s);
+  else
+    fon ? hydro_w<Q, S, KIND, false, true>(wrap, a, grid, s) : hydro_w<Q, S, KIND, false, false>(wrap, a, grid, s);
   return hipGetLastError();
 }
 
