@@ -21,6 +21,9 @@
 // Bytes per fluid cell: Q S + 4 (mask) + 24 in the first pass; 4 + 24 + the
 // neighbours' velocities (mostly from L2) + 4 in the second, 24 + 4 inside the
 // step.  Per solid cell 4 in the first pass (nothing is stored), 8 in the second.
+#include <cstdlib>
+#include <type_traits>
+
 #include "lbm_device.hpp"
 #include "lbm_internal.hpp"
 #include "lbm_scalar.hpp"
@@ -40,18 +43,17 @@ struct WaleOut {
   uint32_t* stats;    // null or [clipped cells, bits of the largest raw nu_t]
 };
 
-// fp32 populations of the first pass are loaded non-temporally: each is read
-// once, and the L2 is left to the velocity planes (256^3 D3Q27 0.417 -> 0.365
-// ms; the step after it reads its populations from memory again either way).
-// 16-bit ones are faster through L2, whose lines two neighbouring odd-state
-// tiles share (512^3 fp16 2.07 -> 1.86 ms, with a scalar 3.48 -> 3.20).
-template <int Q, typename S, int q>
+// NT: the first pass loads its populations non-temporally (wale_nt).
+template <int Q, typename S, int q, bool NT>
 __device__ __forceinline__ float read_pop_once(const S* base, size_t ps, const Nbr& nb, uint32_t i, uint32_t m,
                                                bool odd) {
-  if constexpr (sizeof(S) == 4) {
+  if constexpr (NT) {
     const bool own = !odd || ((m >> q) & 1u);
     const uint32_t j = own ? i : i + (uint32_t)nb.template off<-lat_c(q, 0), -lat_c(q, 1), -lat_c(q, 2)>();
-    return __builtin_nontemporal_load(base + (size_t)(own ? q : lat_opp(q)) * ps + j);
+    using Raw = std::conditional_t<sizeof(S) == 4, float, uint16_t>;
+    const Raw raw = __builtin_nontemporal_load((const Raw*)(base + (size_t)(own ? q : lat_opp(q)) * ps + j));
+    const S v = __builtin_bit_cast(S, raw);
+    return pop_ld<S, Q, q>(&v, 0);
   } else {
     return read_pop<Q, S, q>(base, ps, nb, i, m, odd);
   }
@@ -64,9 +66,12 @@ __device__ __forceinline__ float read_pop_once(const S* base, size_t ps, const N
 // wall velocity).  With QS the pass takes the previous step's passive-scalar
 // step along (no axis wraps then): it collides with exactly these velocities,
 // so its own read of the populations (Q S bytes per cell) is saved.
-template <int Q, typename S, bool WRAP, int QS>
-__global__ __launch_bounds__(256) void k_wale_local(WaleFields a, uint32_t deal, ScalarStepArgs sc) {
-  const uint32_t i = xcd_remap(blockIdx.x, gridDim.x, deal) * 256 + threadIdx.x;
+// Blocks in the plain order: against stretches and runs per XCD (xcd_remap) the
+// best or within 1 % of it at every size measured, 3 to 7 % better for large
+// fp32 domains (512^3 tank 8.52 -> 7.93 ms per step with the loads of wale_nt).
+template <int Q, typename S, bool WRAP, int QS, bool NT>
+__global__ __launch_bounds__(256) void k_wale_local(WaleFields a, ScalarStepArgs sc) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= a.d.N) return;
   float* const vel = a.work;
   float* const strain = a.work + 3 * a.ps;
@@ -79,7 +84,7 @@ __global__ __launch_bounds__(256) void k_wale_local(WaleFields a, uint32_t deal,
   if constexpr (QS > 0) scalar_load<QS>(sc, i, hv);
   sfor<0, Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    fv[q] = read_pop_once<Q, S, q>((const S*)a.f, a.d.ps, nb, i, m, a.odd != 0);
+    fv[q] = read_pop_once<Q, S, q, NT>((const S*)a.f, a.d.ps, nb, i, m, a.odd != 0);
   });
   float Fm[3] = {a.p.F[0], a.p.F[1], a.p.F[2]};
   bool fon = a.p.force_on != 0;
@@ -266,24 +271,41 @@ static uint32_t wale_zlen(const Dom& d) {
   return z;
 }
 
-template <int Q, typename S>
-static void local_q(const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
+// Whether the first pass's population loads are non-temporal: they keep the
+// velocity planes in the caches for the pass that follows, which pays while the
+// populations are a few times the last-level cache.  Below that they would be
+// found in it by the step; far above, ordinary loads stream better.  ms per
+// step with the closure, plain loads -> non-temporal, by bytes of populations:
+//   tanks D3Q27 fp32 128^3 (0.23 GB) 0.175 -> 0.182, 200^3 (0.86) 0.650 -> 0.613,
+//     256^3 (1.81) 1.170 -> 1.167, 320^3 2.17 -> 2.29, 512^3 7.93 -> 8.34;
+//     fp16 128^3 (0.11) 0.145 -> 0.157, 200^3 (0.43) 0.446 -> 0.437, 320^3 (1.77)
+//     1.45 -> 1.52, 512^3 5.17 -> 5.42
+//   periodic D3Q27 fp32 192^3 (0.76) 0.581 -> 0.527, D3Q19 bf16 256^3 (0.64) 0.681
+//     -> 0.668, open D3Q19 384 x 128 x 128 fp32 (0.48) 0.421 -> 0.366, fp16 (0.24)
+//     0.276 -> 0.262
+// LBM_WALE_NT=0 or 1 overrides it (tuning); any choice gives the same values.
+static bool wale_nt(int Q, size_t elem, const Dom& d) {
+  if (const char* e = getenv("LBM_WALE_NT"))
+    if (*e) return e[0] == '1';
+  const size_t bytes = (size_t)Q * elem * d.N;
+  return bytes > 230000000 && bytes < 1500000000;
+}
+
+template <int Q, typename S, bool NT>
+static void local_n(const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
   const dim3 grid((a.d.N + 255) / 256), block(256);
-  // One stretch per XCD while populations, mask and the six planes fit the
-  // last-level cache (256 MiB), short runs beyond (xcd_remap).  Whole step of a
-  // closed D3Q27 cavity, stretch -> dealt ms: fp16 144^3 (245 MB) 0.1455 -> 0.1472,
-  // 152^3 (288) 0.1864 -> 0.1833, 192^3 0.405 -> 0.388; fp32 128^3 (285) 0.1458 ->
-  // 0.1460, with a tracer taken along 0.172 -> 0.174, 136^3 (342) 0.182 -> 0.179,
-  // 192^3 0.604 -> 0.578, 320^3 2.875 -> 2.867.
-  const size_t bytes = ((size_t)Q * sizeof(S) + 28) * a.d.N;
-  const uint32_t deal = bytes < 270000000 ? kXcdStretch : 5u;
   const ScalarStepArgs none{};
   if (sc)
-    hipLaunchKernelGGL((k_wale_local<Q, S, false, 7>), grid, block, 0, s, a, deal, *sc);
+    hipLaunchKernelGGL((k_wale_local<Q, S, false, 7, NT>), grid, block, 0, s, a, *sc);
   else if (a.d.per[0] || a.d.per[1] || a.d.per[2] || a.open)
-    hipLaunchKernelGGL((k_wale_local<Q, S, true, 0>), grid, block, 0, s, a, deal, none);
+    hipLaunchKernelGGL((k_wale_local<Q, S, true, 0, NT>), grid, block, 0, s, a, none);
   else
-    hipLaunchKernelGGL((k_wale_local<Q, S, false, 0>), grid, block, 0, s, a, deal, none);
+    hipLaunchKernelGGL((k_wale_local<Q, S, false, 0, NT>), grid, block, 0, s, a, none);
+}
+
+template <int Q, typename S>
+static void local_q(const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {
+  wale_nt(Q, sizeof(S), a.d) ? local_n<Q, S, true>(a, sc, s) : local_n<Q, S, false>(a, sc, s);
 }
 
 hipError_t launch_wale_local(int Q, int storage, const WaleFields& a, const ScalarStepArgs* sc, hipStream_t s) {

@@ -143,3 +143,37 @@ def test_tank_with_body_follows_the_oracle(Q, collision):
     fl = tc["solid"] == 0
     assert np.abs(s.populations()[:, fl].astype(np.float64) - o.get_f()[:, fl]).max() < 2e-6
     s.close()
+
+
+@pytest.mark.parametrize("kind", ["closed", "periodic", "tracer"])
+@pytest.mark.parametrize("Q,collision,storage", [(27, "cm", "f32"), (19, "trt", "f32"), (27, "trt", "f16"),
+                                                 (19, "bgk", "bf16")])
+def test_loads_of_the_velocity_pass_give_the_same_bits(kind, Q, collision, storage, monkeypatch):
+    """The velocity pass with ordinary and with non-temporal population loads,
+    both parities: the choice goes by the domain's size."""
+    dims = (19, 13, 9)
+    out = []
+    for nt in ("0", "1"):
+        monkeypatch.setenv("LBM_WALE_NT", nt)
+        if kind == "periodic":
+            solid = np.zeros((9, 13, 19), np.uint8)
+            solid[3:5, 4, 6:8] = 1
+            s = L.Solver(Q, dims, nu=0.004, collision=collision, storage=storage, periodic=(True,) * 3,
+                         solid=solid.reshape(-1))
+            s.init_with(*cases.tgv_field(dims, 0.03))
+        else:
+            s, _ = cavity(Q, collision, storage, dims)
+        if kind == "tracer":
+            k = s.enable_scalar_distribution(0.01, "d3q7")
+            s.set_scalar_concentration(k, np.linspace(0.0, 1.0, s.n, dtype=np.float32))
+        s.set_wale(True)
+        s.run(1)
+        a = [s.omega_field()]
+        s.run(4)
+        a += [s.omega_field(), s.populations()]
+        if kind == "tracer":
+            a.append(s.gather_scalar_concentration(k))
+        out.append(a)
+        s.close()
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
