@@ -112,6 +112,8 @@ typedef struct lbm_ibm_diag {
 /* ---- context ------------------------------------------------------------ */
 /* No reference counterpart (wgpu device creation, gpu/backend.rs:1895+). */
 int lbm_ctx_create(int device, lbm_ctx** out);
+/* Domains and batches still alive keep what they use of the context: it is
+ * given back with the last of them. */
 void lbm_ctx_destroy(lbm_ctx* ctx);
 const char* lbm_last_error(const lbm_ctx* ctx);
 /* Backend capability probes, backend.rs:157-199. */

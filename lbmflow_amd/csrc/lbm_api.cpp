@@ -31,7 +31,20 @@ struct lbm_ctx {
   hipStream_t stream = nullptr;
   std::string err;
   Readback rb;
+  // domains and batches on it; the last one to go after lbm_ctx_destroy takes
+  // the context along
+  int users = 0;
+  bool closed = false;
 };
+
+static void ctx_delete(lbm_ctx* ctx) {
+  if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+  delete ctx;
+}
+
+static void ctx_release(lbm_ctx* ctx) {
+  if (--ctx->users == 0 && ctx->closed) ctx_delete(ctx);
+}
 
 struct lbm_fields {
   lbm_ctx* ctx = nullptr;
@@ -628,8 +641,8 @@ int lbm_ctx_create(int device, lbm_ctx** out) {
 
 void lbm_ctx_destroy(lbm_ctx* ctx) {
   if (!ctx) return;
-  if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-  delete ctx;
+  ctx->closed = true;
+  if (ctx->users == 0) ctx_delete(ctx);
 }
 
 const char* lbm_last_error(const lbm_ctx* ctx) { return ctx ? ctx->err.c_str() : "null context"; }
@@ -721,6 +734,7 @@ int lbm_fields_alloc(lbm_ctx* ctx, int Q, int storage, const int dims[3], const 
   lbm_fields* fl = new (std::nothrow) lbm_fields();
   if (!fl) return LBM_ERR_NOMEM;
   fl->ctx = ctx;
+  ++ctx->users;
   fl->Q = Q;
   fl->storage = storage;
   fl->d.nx = dims[0];
@@ -804,7 +818,9 @@ void lbm_fields_free(lbm_fields* fl) {
     if (fl->prof[k]) (void)hipFree(fl->prof[k]);
   }
   for (auto& pa : fl->pr_allocs) (void)hipFree(pa.first);
+  lbm_ctx* ctx = fl->ctx;
   delete fl;
+  ctx_release(ctx);
 }
 
 size_t lbm_fields_device_bytes(const lbm_fields* fl) { return fl ? fl->bytes : 0; }
@@ -2219,6 +2235,7 @@ int lbm_batch_create(lbm_ctx* ctx, lbm_fields* const* members, int n, lbm_batch*
   lbm_batch* b = new (std::nothrow) lbm_batch();
   if (!b) return LBM_ERR_NOMEM;
   b->ctx = ctx;
+  ++ctx->users;
   b->Q = f0->Q;
   b->storage = f0->storage;
   b->collision = f0->collision;
@@ -2287,7 +2304,9 @@ void lbm_batch_destroy(lbm_batch* b) {
   if (b->ibm) ibm_destroy(b->ibm);
   for (void* p : {(void*)b->tab, (void*)b->ent, (void*)b->cells, b->ring, (void*)b->ring_pos})
     if (p) (void)hipFree(p);
+  lbm_ctx* ctx = b->ctx;
   delete b;
+  ctx_release(ctx);
 }
 
 int lbm_batch_info(const lbm_batch* b, int* members, uint32_t* tiles, uint32_t* forced_cells, uint32_t* grid) {

@@ -61,3 +61,25 @@ def test_small_domain_holds_little_device_memory():
     s.populations()
     assert before - free_bytes() <= 8 << 20
     s.close()
+
+
+def test_a_context_closed_first_serves_its_domains():
+    """At interpreter exit a context can be finalized before the solvers and
+    batches on it: they keep what they use of it until the last of them goes."""
+    import lbmflow_amd as L
+
+    ctx = L.Context(0)
+    s = []
+    for n in (12, 14):
+        s.append(L.Solver(19, (n,) * 3, nu=0.05, ctx=ctx))
+        s[-1].build_wall_rims([1] * 6, np.eye(6, 3) * 0.02)
+    b = L.Batch(s)
+    ctx.close()
+    b.run(2)
+    rho = s[0].moments()[0]
+    assert np.all(np.isfinite(rho)) and s[1].time == 2
+    s[0].close()
+    b.close()
+    s[1].run(1)
+    assert s[1].populations().shape == (19, 14 ** 3)
+    s[1].close()
