@@ -713,6 +713,28 @@ hipError_t launch_stream_copy(const void* a, void* b, size_t bytes, hipStream_t 
   return hipGetLastError();
 }
 
+// Into pinned memory, 16 bytes per lane where both ends allow it (dst is a slot
+// or a place in it, src any array): bound by the host link.
+template <typename T>
+__global__ __launch_bounds__(256) void k_to_host(T* dst, const T* src, size_t n) {
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+}
+
+hipError_t launch_to_host(void* dst, const void* src, size_t n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (((uintptr_t)dst | (uintptr_t)src | n) % 16 == 0) {
+    const size_t v = n / 16;
+    hipLaunchKernelGGL((k_to_host<uint4>), dim3((unsigned)std::min<size_t>((v + 255) / 256, 512)), dim3(256), 0, s,
+                       (uint4*)dst, (const uint4*)src, v);
+  } else {
+    const size_t v = n / 4;
+    hipLaunchKernelGGL((k_to_host<uint32_t>), dim3((unsigned)std::min<size_t>((v + 255) / 256, 2048)), dim3(256), 0,
+                       s, (uint32_t*)dst, (const uint32_t*)src, v);
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_fill_f32(float* p, size_t n, float v, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_fill, dim3(blocks_for(n)), dim3(256), 0, s, p, n, v);

@@ -4,7 +4,10 @@
 // moves it through its own staging on one thread, which also takes the fresh
 // pages' faults (10 GB/s measured, 207 ms for the four moment fields of 512^3
 // cells).  Here the device writes 2 MiB pinned slots at the link's rate and a
-// few threads copy them out, so the faults and the copies run in parallel.
+// few threads copy them out, so the faults and the copies run in parallel.  A
+// kernel writes the slots: the runtime's copies go to a DMA engine of its
+// choice, and now and then, for a while, to one that takes 166 us per slot
+// instead of 42 (32 MB 1.0 or 3.0 ms).
 // Results are produced piece by piece through a bounded device workspace, so
 // no call allocates a full-size array either.
 //
@@ -29,6 +32,9 @@
 
 namespace lbm {
 
+// n bytes (a multiple of 4, 4-byte aligned) into pinned memory (lbm_kernels.hip)
+hipError_t launch_to_host(void* dst, const void* src, size_t n, hipStream_t s);
+
 class Readback {
  public:
   struct Seg {
@@ -40,6 +46,9 @@ class Readback {
   static constexpr int kSlots = 24;
   static constexpr size_t kWorkBytes = (size_t)64 << 20;
   static constexpr size_t kMinWorkBytes = (size_t)64 << 10;
+  // a small array that no kernel has just written is 3 us faster by the runtime's
+  // copy (110 KB 12.1 against 15.4 us)
+  static constexpr size_t kSmallCopy = (size_t)512 << 10;
   static constexpr int kThreads = 12;  // of the 16 host cores a GPU comes with
 
   Readback() = default;
@@ -113,7 +122,8 @@ class Readback {
         for (size_t a = 0, b; a < segs.size() && e == hipSuccess; a = b) {
           size_t n = 0;
           for (b = a; b < segs.size() && segs[b].src == (const char*)segs[a].src + n; ++b) n += segs[b].bytes;
-          e = hipMemcpyAsync(pin_ + at, segs[a].src, n, hipMemcpyDeviceToHost, s);
+          e = segs.size() == 1 && n <= kSmallCopy ? hipMemcpyAsync(pin_ + at, segs[a].src, n, hipMemcpyDeviceToHost, s)
+                                                  : launch_to_host(pin_ + at, segs[a].src, n, s);
           at += n;
         }
         const hipError_t w = hipStreamSynchronize(s);
@@ -135,15 +145,15 @@ class Readback {
         }
       }
       // one copy per slot, over as many segments as lie together in the
-      // source: a copy costs the caller up to 45 us whatever its size (populations
-      // of 24^3 cells, 19 planes of 55 KB: 1.03 -> 0.07 ms)
+      // source (a DMA copy for each of 19 planes of 24^3 cells took 1.03 ms, one
+      // for all 0.07)
       Item it;
       const char* src = nullptr;
       size_t fill = 0;
       auto flush = [&] {
         if (fill == 0 || e != hipSuccess) return;
         it.slot = job.take(pool.empty() ? this : nullptr);
-        e = hipMemcpyAsync(pin_ + (size_t)it.slot * kSlotBytes, src, fill, hipMemcpyDeviceToHost, s);
+        e = launch_to_host(pin_ + (size_t)it.slot * kSlotBytes, src, fill, s);
         if (e == hipSuccess) e = hipEventRecord(ev_[it.slot], s);
         if (e == hipSuccess) job.put(it);
         fill = 0;
@@ -266,10 +276,10 @@ class Readback {
     if (slots_ >= n) return true;
     if (refused_ && n >= refused_) return false;
     void* p = nullptr;
-    bool ok = hipHostMalloc(&p, kSlotBytes * n, hipHostMallocDefault) == hipSuccess;
+    bool ok = hipHostMalloc(&p, kSlotBytes * n, hipHostMallocCoherent) == hipSuccess;
     while (ok && n > 1 && (int)ev_.size() < n) {
       hipEvent_t e;
-      ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+      ok = hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) == hipSuccess;
       if (ok) ev_.push_back(e);
     }
     if (!ok) {
