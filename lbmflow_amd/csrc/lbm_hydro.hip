@@ -882,7 +882,7 @@ __global__ __launch_bounds__(256) void k_hydro(HydroArgs a) {
 // under the populations' loads.  Four waves per SIMD as k_hydro has.
 // Per step, closure and collide-stream: 256^3 D3Q27 fp32 1.153 -> 1.094 ms (the
 // velocity pass 0.365, this kernel 0.705 / 0.753); 512^3 fp16 with a D3Q7
-// tracer taken along by that pass 8.31 -> 6.62 ms (3.20, and 3.13 / 3.70 here,
+// tracer taken along by that pass 8.31 -> 6.41 ms (3.10, and 3.03 / 3.58 here,
 // where nu_t's 380 VALU instructions per wave make it VALU-bound).
 template <int Q, typename S, int KIND, bool ODD>
 __global__ __launch_bounds__(256, 4) void k_hydro_wale(HydroArgs a) {
